@@ -1,6 +1,8 @@
 // Launches of the grouped GEMM kernel (mgg_gemm_kernel.h) for N even: the
 // instances every even N runs, bf16/fp16 with N-major and K-major B, fused
 // epilogues, gathered A, and fp8.  Odd N goes to mgg_gemm_odd.hip.
+#include <type_traits>
+
 #include "mgg_gemm_kernel.h"
 
 namespace mgg {
@@ -21,9 +23,8 @@ int launch_typed(int block_m, int block_n, const GemmParams& p, int workers, hip
   // rows) and as many stages as the LDS budget holds, except the 256x256
   // tile (see MGG_SBK256).  Fused epilogues are compiled for the 256x256 and
   // 128x128 tiles (two 32-column blocks per wave).
-  constexpr int kSbk256 = T::kBKMajor ? MGG_KM_SBK256 : MGG_SBK256;
-  constexpr int kNs256 = T::kBKMajor ? MGG_KM_NS256 : MGG_NS256;
-  MGG_CASE(256, 256, kSbk256, kNs256, MGG_NW256)
+  // K-major B's 256x256 tile is mgg_gemm_kmajor.h's.
+  if constexpr (!T::kBKMajor) { MGG_CASE(256, 256, MGG_SBK256, MGG_NS256, MGG_NW256) }
   MGG_CASE(128, 128, 64, 4, 4)
   if constexpr (EPI == kEpiNone) {
     MGG_CASE(256, 128, 64, 3, 4)
@@ -86,6 +87,12 @@ int launch_epi(int epilogue, int block_m, int block_n, const GemmParams& p, int 
     }
   } else {
     if (p.a_rows != nullptr) return set_error(MGG_ERR_UNSUPPORTED, "gathered A needs N-major 16-bit B");
+  }
+  if constexpr (T::kBKMajor) {
+    if (block_m == 256 && block_n == 256)
+      return launch_kmajor_256(std::is_base_of_v<Bf16, T> ? MGG_DTYPE_BF16 | MGG_B_KMAJOR
+                                                          : MGG_DTYPE_FP16 | MGG_B_KMAJOR,
+                               epilogue, p, workers, stream);
   }
   switch (epilogue) {
     case kEpiNone: return launch_typed<T, kEpiNone>(block_m, block_n, p, workers, stream);

@@ -98,6 +98,8 @@ unsigned long long* clock_probe();
 // `stream` with `workers` workgroups.  Returns MGG_OK or an error code.
 int launch_grouped_gemm(int dtype, int epilogue, int block_m, int block_n, const GemmParams& p,
                         int workers, hipStream_t stream);
+// 256x256 tiles with K-major 16-bit B and even N (dtype with MGG_B_KMAJOR).
+int launch_kmajor_256(int dtype, int epilogue, const GemmParams& p, int workers, hipStream_t stream);
 // The same for odd N (p.n odd), on the tiles compiled for it: 256x256 and
 // 128x128, and 128x512 for 16-bit types without a fused epilogue; other
 // requested tiles compute on the nearest of these.
