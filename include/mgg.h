@@ -379,6 +379,17 @@ int mgg_gather_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token
                     int64_t ld_out, void* stream);
 
 /*
+ * mgg_gather_rows over a whole dispatch layout (num_tokens * top_k rows, of
+ * x's first num_tokens rows), given both of its index arrays: slot_position
+ * and token_index must be the two directions of one mapping, as
+ * mgg_dispatch_layout writes them.  Same result; either array is used,
+ * whichever moves fewer bytes.
+ */
+int mgg_permute_rows(int dtype, const void* x, int64_t ld_x, const int32_t* slot_position,
+                     const int32_t* token_index, const int32_t* num_rows, int64_t num_tokens,
+                     int top_k, int64_t hidden, void* out, int64_t ld_out, void* stream);
+
+/*
  * out[t, :] = sum_{j < top_k, slot_position[t*top_k+j] >= 0}
  *             weights[t*top_k+j] * y[slot_position[t*top_k+j], :]
  * for t < num_tokens: fp32 accumulation in slot order, one rounding to the

@@ -820,6 +820,21 @@ int mgg_gather_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token
                                  static_cast<hipStream_t>(stream));
 }
 
+int mgg_permute_rows(int dtype, const void* x, int64_t ld_x, const int32_t* slot_position,
+                     const int32_t* token_index, const int32_t* num_rows, int64_t num_tokens,
+                     int top_k, int64_t hidden, void* out, int64_t ld_out, void* stream) {
+  mgg::clear_error();
+  if (num_tokens < 0 || top_k < 0) return set_error(MGG_ERR_INVALID, "sizes must be >= 0");
+  const int64_t max_rows = num_tokens * top_k;
+  // One slot a token: nothing is read twice, and the gather's writes are in order.
+  if (top_k > 1 && (dtype == MGG_DTYPE_BF16 || dtype == MGG_DTYPE_FP16) && max_rows > 0 &&
+      hidden > 0 && ld_x >= hidden && ld_out >= hidden && x != nullptr && slot_position != nullptr &&
+      out != nullptr && mgg::scatter_rows_supported(x, ld_x, hidden, 2, out, ld_out))
+    return mgg::launch_scatter_rows(x, ld_x, slot_position, num_tokens, top_k, max_rows, hidden, 2,
+                                    out, ld_out, static_cast<hipStream_t>(stream));
+  return mgg_gather_rows(dtype, x, ld_x, token_index, num_rows, max_rows, hidden, out, ld_out, stream);
+}
+
 int mgg_combine_rows(int dtype, const void* y, int64_t ld_y, const int32_t* slot_position,
                      const float* weights, int64_t num_tokens, int top_k, int64_t hidden,
                      void* out, int64_t ld_out, void* stream) {

@@ -322,6 +322,38 @@ gather_rows_kernel(const uint8_t* x, int64_t ld_x, const int32_t* token_index,
   }
 }
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// out[slot_pos[t, j], :] = x[t, :] for the slots with a position in
+// [0, rows_max): the gather above by its inverse, so a token's row is read
+// once and written top_k times, where the gather reads it from the far caches
+// top_k times.  One 16-byte chunk of one token per thread (blockIdx.y: which
+// kRowThreads chunks of the row), so every row's stores are in flight at once.
+// Bound by the writes.  Measured (T = 4096, top-8, H = 7168, 470 MB written):
+// gather 140.3 us, this 93.9 us (one box, kernel trace); the non-temporal hint for
+// outputs past the last-level cache's reach (kStreamBytes).
+template <bool NT>
+__global__ void __launch_bounds__(kRowThreads)
+scatter_rows_kernel(const uint8_t* x, int64_t ld_x_bytes, const int32_t* slot_pos,
+                    int64_t num_tokens, int32_t top_k, int64_t rows_max, int64_t chunks,
+                    uint8_t* out, int64_t ld_out_bytes) {
+  const int64_t c = (int64_t)blockIdx.y * kRowThreads + threadIdx.x;
+  if (c >= chunks) return;
+  for (int64_t t = blockIdx.x; t < num_tokens; t += gridDim.x) {
+    const u32x4 v = reinterpret_cast<const u32x4*>(x + t * ld_x_bytes)[c];
+    const int32_t* pos_t = slot_pos + t * top_k;
+    for (int j = 0; j < top_k; ++j) {
+      const int64_t pos = pos_t[j];
+      if (pos < 0 || pos >= rows_max) continue;
+      u32x4* dst = reinterpret_cast<u32x4*>(out + pos * ld_out_bytes) + c;
+      if constexpr (NT)
+        __builtin_nontemporal_store(v, dst);
+      else
+        *dst = v;
+    }
+  }
+}
+
 template <class T>
 struct Elem;
 template <>
@@ -352,7 +384,6 @@ struct Elem<_Float16> {
 // at a time with plain loads (5.0 against 4.5 TB/s), at top-2 (H = 2048,
 // 6.1 TB/s with GROUP = 1) 9.5% slower, so the launch takes GROUP = 1 up to
 // two slots per token.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <class T, bool VEC, int GROUP>
 __global__ void __launch_bounds__(kRowThreads)
@@ -415,6 +446,10 @@ combine_rows_kernel(const uint16_t* y, int64_t ld_y, const int32_t* slot_pos,
     }
   }
 }
+
+// Row movement that writes more than this does not find it in the last-level
+// cache (256 MiB) again: its stores go with the non-temporal hint.
+constexpr int64_t kStreamBytes = (int64_t)128 << 20;
 
 int grid_for(int64_t rows) {
   const int64_t g = rows < 1 ? 1 : rows;
@@ -501,6 +536,30 @@ int launch_gather_rows(const void* x, int64_t ld_x, const int32_t* token_index,
   if (hipError_t err = hipGetLastError(); err != hipSuccess)
     return hip_error(err, "gather launch");
   return MGG_OK;
+}
+
+int launch_scatter_rows(const void* x, int64_t ld_x, const int32_t* slot_pos, int64_t num_tokens,
+                        int top_k, int64_t rows_max, int64_t hidden, int elem_bytes, void* out,
+                        int64_t ld_out, hipStream_t stream) {
+  if (num_tokens <= 0 || top_k <= 0 || rows_max <= 0 || hidden <= 0) return MGG_OK;
+  const int64_t chunks = hidden * elem_bytes / 16;
+  const dim3 grid((unsigned)grid_for(num_tokens), (unsigned)((chunks + kRowThreads - 1) / kRowThreads));
+#define MGG_SCATTER(NT_)                                                                        \
+  hipLaunchKernelGGL(scatter_rows_kernel<NT_>, grid, dim3(kRowThreads), 0, stream,              \
+                     (const uint8_t*)x, ld_x * elem_bytes, slot_pos, num_tokens, top_k, rows_max, \
+                     chunks, (uint8_t*)out, ld_out * elem_bytes)
+  if (rows_max * hidden * elem_bytes > kStreamBytes) MGG_SCATTER(true); else MGG_SCATTER(false);
+#undef MGG_SCATTER
+  if (hipError_t err = hipGetLastError(); err != hipSuccess)
+    return hip_error(err, "scatter launch");
+  return MGG_OK;
+}
+
+bool scatter_rows_supported(const void* x, int64_t ld_x, int64_t hidden, int elem_bytes,
+                            const void* out, int64_t ld_out) {
+  const int64_t row_bytes = hidden * elem_bytes;
+  return row_bytes % 16 == 0 && (ld_x * elem_bytes) % 16 == 0 && (ld_out * elem_bytes) % 16 == 0 &&
+         aligned16(x) && aligned16(out) && row_bytes / 16 <= 65535LL * kRowThreads;
 }
 
 namespace {

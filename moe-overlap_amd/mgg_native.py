@@ -103,6 +103,10 @@ _SIGNATURES = {
     "mgg_gather_rows": [
         _c_i32, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr,
     ],
+    "mgg_permute_rows": [
+        _c_i32, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr,  # dtype, x, ld_x, slot_pos, token_index, num_rows
+        _c_i64, _c_i32, _c_i64, _c_ptr, _c_i64, _c_ptr,  # T, top_k, hidden, out, ld_out, stream
+    ],
     "mgg_combine_rows": [
         _c_i32, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i32, _c_i64, _c_ptr, _c_i64, _c_ptr,
     ],
