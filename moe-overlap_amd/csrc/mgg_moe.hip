@@ -193,49 +193,55 @@ layout_scatter_kernel(const In* idx, int64_t A, int32_t top_k, int32_t E, const 
 
 // Pass 3 for up to kMaxWideExperts experts: a chunk's kLayoutChunk
 // assignments take one lane each (kLayoutChunk / 64 waves).  Each wave ranks
-// its 64 assignments per expert with ballots and records its per-expert
-// counts in LDS; a prefix over the waves, per expert, then gives each wave's
-// base.  Positions are those of layout_scatter_kernel (assignment order
-// within each expert), with every assignment in flight at once.
+// its 64 assignments per expert and records its per-expert counts in LDS; a
+// prefix over the waves, per expert, then gives each wave's base.  Positions
+// are those of layout_scatter_kernel (assignment order within each expert),
+// with every assignment in flight at once.
 //
-// kScan (small layouts, nb * E <= kFusedScanMax): pass 2 runs inside this
-// pass instead of as its own launch.  `hist` then holds the count pass's
+// The lanes that share an expert are found bit by bit: one ballot per bit of
+// the expert number (8 for 256 experts, where a round per distinct expert of
+// the 64 takes about 57).
+//
+// kLayoutTable (small layouts, nb * E <= kFusedScanMax): pass 2 runs inside
+// this pass instead of as its own launch.  `hist` then holds the count pass's
 // per-chunk counts as they are, and every workgroup derives its chunk's base
 // per expert from them: offsets[e] (an exclusive scan of the expert totals
 // over the whole table) plus the counts of the chunks before its own.
-// Workgroup 0 also writes counts and offsets.  The positions are the same.
+// Workgroup 0 also writes counts and offsets.  The table is read by as many
+// (part, expert) threads as the counters' LDS has room to add up: latency
+// bounds it.
+//
+// kLayoutOne (a single chunk, decode steps): the expert totals are this
+// workgroup's own counts, so there is no count pass either, one launch in all.
+//
+// Measured (kernel trace): T = 4096, top-8, 256 experts 12.8 -> 5.9 us; 32
+// tokens, top-2, 16 experts 4.5 + 4.9 us in two launches -> 5.2 in one.
+enum LayoutScan { kLayoutBases, kLayoutTable, kLayoutOne };
 constexpr int kWideWaves = kLayoutChunk / 64;
 constexpr int kMaxWideExperts = 1024;  // [kWideWaves][E] int32 counters in 64 KiB of LDS
 constexpr int64_t kFusedScanMax = 16384;  // table entries every workgroup reads (64 KiB)
 
-template <class In, bool kScan>
+template <class In, LayoutScan kScan>
 __global__ void __launch_bounds__(kLayoutChunk)
 layout_scatter_wide_kernel(const In* idx, int64_t A, int32_t top_k, int32_t E,
                            const int32_t* hist, int32_t nb, int32_t* counts, int32_t* offsets,
                            int32_t* slot_pos, int32_t* token_index, int32_t* row_assign) {
   extern __shared__ int32_t s_cnt[];  // [kWideWaves][E]: counts, then bases
-  __shared__ int32_t s_base[kScan ? kMaxWideExperts : 1];  // kScan: chunk base per expert
-  __shared__ int32_t s_wsum[kScan ? kWideWaves : 1];
+  __shared__ int32_t s_base[kScan != kLayoutBases ? kMaxWideExperts : 1];  // chunk base per expert
+  __shared__ int32_t s_wsum[kScan != kLayoutBases ? kWideWaves : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = tid >> 6;
-  if constexpr (kScan) {
-    // Thread x < E: expert x's total over all chunks and over the chunks
-    // before this one; then an exclusive scan of the totals (within each
-    // wave by shuffles, then over the wave sums).
-    int32_t total = 0, before = 0;
-    if (tid < E) {
-      for (int b0 = 0; b0 < nb; b0 += 8) {  // eight chunks' loads in flight at a time
-        int32_t c[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) c[j] = b0 + j < nb ? hist[(int64_t)(b0 + j) * E + tid] : 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          if (b0 + j < (int)blockIdx.x) before += c[j];
-          total += c[j];
-        }
-      }
-    }
+  const int64_t a = (int64_t)blockIdx.x * kLayoutChunk + tid;
+  int32_t e = -1;
+  if (a < A) {
+    const int64_t v = (int64_t)idx[a];
+    e = (v >= 0 && v < E) ? (int32_t)v : -1;
+  }
+  // Thread x < E holds expert x's total over all chunks (and `before`, the
+  // chunks before this one): an exclusive scan of the totals, within each
+  // wave by shuffles, then over the wave sums.
+  auto scan_totals = [&](int32_t total, int32_t before) {
     int32_t incl = total;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -255,30 +261,61 @@ layout_scatter_wide_kernel(const In* idx, int64_t A, int32_t top_k, int32_t E,
         if (tid == E - 1) offsets[E] = off + total;
       }
     }
+  };
+  if constexpr (kScan == kLayoutTable) {
+    // Up to kWideWaves / 2 parts per expert: two sums each fit s_cnt.
+    int parts = kLayoutChunk / E;
+    parts = parts < kWideWaves / 2 ? parts : kWideWaves / 2;
+    const int part = tid / E, x = tid - part * E;
+    if (part < parts) {
+      int32_t total = 0, before = 0;
+      for (int b0 = part; b0 < nb; b0 += 8 * parts) {  // eight chunks' loads in flight at a time
+        int32_t c[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int bj = b0 + j * parts;
+          c[j] = bj < nb ? hist[(int64_t)bj * E + x] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if (b0 + j * parts < (int)blockIdx.x) before += c[j];
+          total += c[j];
+        }
+      }
+      s_cnt[2 * part * E + x] = total;
+      s_cnt[(2 * part + 1) * E + x] = before;
+    }
+    __syncthreads();
+    int32_t total = 0, before = 0;
+    if (tid < E) {
+      for (int q = 0; q < parts; ++q) {
+        total += s_cnt[2 * q * E + tid];
+        before += s_cnt[(2 * q + 1) * E + tid];
+      }
+    }
+    scan_totals(total, before);  // its barrier: every sum has been read
   }
   for (int i = tid; i < kWideWaves * E; i += kLayoutChunk) s_cnt[i] = 0;
   __syncthreads();
-  const int64_t a = (int64_t)blockIdx.x * kLayoutChunk + tid;
-  int32_t e = -1;
-  if (a < A) {
-    const int64_t v = (int64_t)idx[a];
-    e = (v >= 0 && v < E) ? (int32_t)v : -1;
-  }
   const bool valid = e >= 0;
-  uint64_t todo = __ballot(valid);
-  int32_t rank = 0;
-  while (todo != 0) {
-    const int leader = __builtin_ctzll(todo);
-    const int32_t el = __builtin_amdgcn_readlane(e, leader);
-    const bool mine = valid && e == el;
-    const uint64_t m = __ballot(mine);
-    if (mine) rank = __builtin_popcountll(m & ((1ull << lane) - 1ull));
-    if (lane == leader) s_cnt[w * E + el] = __builtin_popcountll(m);
-    todo &= ~m;
+  uint64_t same = __ballot(valid);
+  for (int bit = 1; bit < E; bit <<= 1) {  // uniform
+    const bool set = (e & bit) != 0;
+    const uint64_t m = __ballot(set);
+    same &= set ? m : ~m;
   }
+  const int32_t rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+  if (valid && rank == 0) s_cnt[w * E + e] = __builtin_popcountll(same);
   __syncthreads();
+  if constexpr (kScan == kLayoutOne) {
+    int32_t total = 0;
+    if (tid < E)
+      for (int v = 0; v < kWideWaves; ++v) total += s_cnt[v * E + tid];
+    scan_totals(total, 0);
+    // Thread x writes and then reads s_base[x]: kLayoutChunk covers E.
+  }
   for (int x = tid; x < E; x += kLayoutChunk) {
-    int32_t run = kScan ? s_base[x] : hist[(int64_t)blockIdx.x * E + x];
+    int32_t run = kScan != kLayoutBases ? s_base[x] : hist[(int64_t)blockIdx.x * E + x];
     for (int v = 0; v < kWideWaves; ++v) {
       const int32_t c = s_cnt[v * E + x];
       s_cnt[v * E + x] = run;
@@ -295,6 +332,7 @@ layout_scatter_wide_kernel(const In* idx, int64_t A, int32_t top_k, int32_t E,
     slot_pos[a] = -1;
   }
 }
+static_assert(kMaxWideExperts <= kLayoutChunk, "one thread per expert in the scans");
 
 constexpr int kRowThreads = 256;
 
@@ -469,7 +507,12 @@ int launch_dispatch_layout(const void* topk_idx, int idx_type, int64_t num_token
   const int64_t A = num_tokens * top_k;
   const int64_t nb = layout_chunks(A);
   const size_t lds = (size_t)num_experts * sizeof(int32_t);
-  if (nb > 0) {
+  // Small layouts scan inside the position pass (one launch fewer), and a
+  // single chunk counts there as well.
+  const bool wide = nb > 0 && num_experts > 0 && num_experts <= kMaxWideExperts;
+  const bool one = wide && nb == 1;
+  const bool fused = wide && nb * (int64_t)num_experts <= kFusedScanMax;
+  if (nb > 0 && !one) {
     if (idx_type == MGG_INT64)
       hipLaunchKernelGGL(layout_count_kernel<int64_t>, dim3((unsigned)nb), dim3(kLayoutThreads),
                          lds, stream, (const int64_t*)topk_idx, A, num_experts, hist);
@@ -479,9 +522,6 @@ int launch_dispatch_layout(const void* topk_idx, int idx_type, int64_t num_token
     if (hipError_t err = hipGetLastError(); err != hipSuccess)
       return hip_error(err, "layout count launch");
   }
-  // Small layouts scan inside the position pass (one launch fewer).
-  const bool fused = nb > 0 && num_experts > 0 && num_experts <= kMaxWideExperts &&
-                     nb * (int64_t)num_experts <= kFusedScanMax;
   if (!fused) {
     hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(kLayoutScanThreads), 0, stream, hist,
                        (int32_t)nb, num_experts, counts, offsets);
@@ -496,9 +536,13 @@ int launch_dispatch_layout(const void* topk_idx, int idx_type, int64_t num_token
                      num_experts, hist, (int32_t)nb, counts, offsets, slot_pos, token_index,     \
                      row_assign)
     if (idx_type == MGG_INT64) {
-      if (fused) MGG_WIDE(int64_t, true); else MGG_WIDE(int64_t, false);
+      if (one) MGG_WIDE(int64_t, kLayoutOne);
+      else if (fused) MGG_WIDE(int64_t, kLayoutTable);
+      else MGG_WIDE(int64_t, kLayoutBases);
     } else {
-      if (fused) MGG_WIDE(int32_t, true); else MGG_WIDE(int32_t, false);
+      if (one) MGG_WIDE(int32_t, kLayoutOne);
+      else if (fused) MGG_WIDE(int32_t, kLayoutTable);
+      else MGG_WIDE(int32_t, kLayoutBases);
     }
 #undef MGG_WIDE
     if (hipError_t err = hipGetLastError(); err != hipSuccess)

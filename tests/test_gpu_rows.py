@@ -37,3 +37,28 @@ def test_permute_rows(cuda_device, tokens, experts, top_k, hidden, pad, masked):
     # A layout that holds one direction only goes by token_index.
     one_way = dataclasses.replace(lay, slot_position=None)
     assert torch.equal(mlp.permute_tokens(x, one_way)[:n], want)
+
+
+@pytest.mark.parametrize("tokens,top_k,experts", [
+    (1, 1, 1), (512, 2, 16), (128, 8, 1024),  # one chunk: counted in place
+    (513, 2, 3), (1025, 1, 64),               # two chunks: the table's sums in eight parts
+    (2048, 8, 257), (900, 8, 512), (900, 8, 513), (2048, 8, 1024),  # three, two and one part
+    (20000, 4, 300),                          # past the table: bases from the scan pass
+])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_dispatch_layout_paths(cuda_device, tokens, top_k, experts, dtype):
+    gen = torch.Generator().manual_seed(tokens)
+    idx = torch.randint(-1, experts + 1, (tokens, top_k), generator=gen)  # both ends masked
+    lay = mlp.dispatch_layout(idx.to(dtype).to(cuda_device), experts)
+    flat = idx.flatten()
+    valid = (flat >= 0) & (flat < experts)
+    order = torch.argsort(torch.where(valid, flat, experts), stable=True)[: int(valid.sum())]
+    pos = torch.full_like(flat, -1)
+    pos[order] = torch.arange(order.numel())
+    counts = torch.bincount(flat[valid], minlength=experts)
+    n = order.numel()
+    assert torch.equal(lay.counts.cpu().long(), counts)
+    assert torch.equal(lay.offsets.cpu().long(), torch.cat([counts.new_zeros(1), counts.cumsum(0)]))
+    assert torch.equal(lay.slot_position.cpu().long(), pos)
+    assert torch.equal(lay.row_assignment[:n].cpu().long(), order)
+    assert torch.equal(lay.token_index[:n].cpu().long(), order // top_k)
