@@ -118,7 +118,7 @@ int launch_build_work_queue(const int32_t* offsets, int32_t num_experts, int64_t
                             int block_m, int block_n, int32_t* we, int32_t* wm, int32_t* wn,
                             int32_t num_work, hipStream_t stream);
 
-// Dispatch layout (three kernels; `hist` holds layout_chunks(T*k) * E int32).
+// Dispatch layout (one to three kernels; `hist` holds layout_chunks(T*k) * E int32).
 int64_t layout_chunks(int64_t assignments);
 int launch_dispatch_layout(const void* topk_idx, int idx_type, int64_t num_tokens, int top_k,
                            int32_t num_experts, int32_t* counts, int32_t* offsets,

@@ -18,8 +18,9 @@ Differences, all in arguments that do not change results:
   kernel compiles.  They set the queue whose length the atomic schedule's
   ``work_counter`` reports (W + G, W counted for the requested tile) and the
   keys of ``_build_work_queue``; the kernel itself computes with the fastest
-  compiled tile, 256 x 256 for bf16/fp16 (eight waves, two per SIMD, 32-deep
-  B stages and 64-deep A blocks), or the tile named by the keyword-only
+  compiled tile, 256 x 256 for bf16/fp16 where its tiles fill the chip (eight
+  waves, two per SIMD, 32-deep B stages and 64-deep A blocks) and smaller ones
+  where they leave CUs idle, or the tile named by the keyword-only
   ``kernel_tile``.  Every output element is the same fp32 sum in the same K
   order whatever the tile, so results do not depend on either choice.
 * ``block_k``, ``num_warps``, ``num_stages`` are accepted and ignored: the
@@ -57,6 +58,7 @@ Differences, all in arguments that do not change results:
 from __future__ import annotations
 
 import ctypes
+import math
 import operator
 from typing import List, Optional, Tuple, Union
 
@@ -253,34 +255,60 @@ def _build_work_queue(
 # --------------------------------------------------------------------------
 # grouped GEMM
 # --------------------------------------------------------------------------
+# What a round of one tile per CU costs on each kernel tile, in rounds of
+# 256x256 (see _default_kernel_tile).
+_TILE_ROUND_COST = (((256, 256), 1.0), ((256, 128), 0.7), ((128, 256), 0.7), ((128, 128), 0.5))
+
+
 def _default_kernel_tile(m_total: int, num_experts: int, n_size: int = 4096,
                          workers: int = 256) -> Tuple[int, int]:
-    """128x512 or 256x256, from the average rows per expert (no host sync on
-    the offsets).  Rows of a tile past its expert's end are zero-fill DMAs that
-    read nothing, so a tile's cost follows the memory requests of its valid
-    rows; both tiles hold the same 256 KiB of fp32 accumulators (two waves per
-    SIMD).  With at most 128 rows an expert is one m-tile either way and the
-    wide tile reads its A rows half as often, but each of its tiles takes about
-    1.6 times as long and there are half as many: it is taken when N >= 512 and
-    1.6 x its rounds of `workers` tiles stay under the square tile's rounds.
-    Measured on MI355X (HIP-event medians, atomic, µs): E=256 x 128 rows,
-    K=7168, N=2048 (the reference benchmark's default problem) 1271 against
-    1584 (256x256); E=128 x 32 rows, K=N=4096, 682 against 776; but E=16 x 128
-    rows, K=2048, N=4096 (128 wide tiles for 256 workers) 74.9 against 57.4;
-    E=64 x 128, N=1024, 80.6 against 60.9; E=16 x 192 and x 256 rows 74.7 and
-    80.1 against 63.0 and 68.8.  Among the tiles of at most 256 rows and
-    columns, 256x256 is the fastest at every expert size (E=16, K=2048,
-    N=4096, atomic / striped: 64 rows per expert 57.2 / 52.3 against 128x256
-    63.4 / 54.5 and 128x128 55.4 / 50.9; 128 rows 60.9 / 60.5 against 95.5 /
-    94.6 (128x256); 192 rows 63.2 / 62.4 against 101.2 / 98.5; 256-384 rows
-    101-119 against 140-192)."""
-    if num_experts <= 0 or n_size < 512 or m_total > 128 * num_experts:
+    """The tile whose rounds of `workers` tiles cost least, from the average
+    rows per expert (no host sync on the offsets).  Rows of a tile past its
+    expert's end are zero-fill DMAs that read nothing, so a tile's cost follows
+    its valid rows and its columns; what decides is how far the last round
+    leaves the chip idle.  A round costs, in rounds of 256x256, 1.6 on 128x512
+    (at most 128 rows an expert and N >= 512: it reads A half as often), 0.7 on
+    256x128 and 128x256 and 0.5 on 128x128; with one m-tile an expert either
+    way, 128x256 streams the columns 256x256 does and costs 0.9.  Ties go to the larger tile.  Rows
+    per expert are taken two standard deviations above the average that top-k
+    routing spreads them around, so that a tile edge just above the average is
+    not counted on (128x512 goes by the average itself).
+    Measured on MI355X (HIP-event medians of the call, atomic / striped, µs).
+    Fewer 256x256 tiles than workers: E=8 x 200 rows, K=1024, N=2048 (64
+    tiles) 256x256 36.2 / 35.6, 256x128 25.3 / 24.2, 128x128 20.0 / 18.4; the
+    same at K=7168 95.7 / 174.7, 81.2 / 103.0, 78.4 / 77.1; B as [E, N, K],
+    K=2048 60.5 / 62.8, 38.3 / 36.5, 29.4 / 28.1; E=12, 2222 rows, K=1504,
+    N=2050, fp16 (108 tiles) 48.1 / 47.7, 35.3 / 33.4, 45.9 / 43.5; E=16 x 4
+    rows, K=4096, N=2048 (128) 63.4 / 85.1, 57.9 / 59.8, 55.4 / 53.9.
+    A second round begun: E=24 x 16 rows, K=2048, N=4096 (384) 97.6 / 95.7,
+    94.5 / 93.7, 81.1 / 80.7, 128x256 87.9 / 89.4; E=64 x 16 rows, K=1024,
+    N=1408 (384) 54.8 / 55.1, 56.6 / 54.7, 45.3 / 44.1, 49.7 / 49.7.
+    One m-tile an expert, a full round: E=32 x 16 rows, K=7168, N=2048 (256)
+    192.7 / 181.1 against 128x256 171.3 / 167.7.
+    Rounds full: E=16 x 192 rows, K=2048, N=4096 (256) 256x256 63.2 / 62.4
+    against 128x256 101.2 / 98.5; 256-384 rows 101-119 against 140-192.
+    128x512: E=256 x 128 rows, K=7168, N=2048 1271 against 1584 (256x256);
+    E=128 x 32 rows, K=N=4096, 682 against 776; E=64 x 128, N=1024, 80.6
+    against 60.9."""
+    if num_experts <= 0:
         return 256, 256
-    rows = max(-(-m_total // num_experts), 1)
     w = max(int(workers), 1)
-    rounds_wide = -(-(num_experts * -(-rows // 128) * -(-n_size // 512)) // w)
-    rounds_square = -(-(num_experts * -(-rows // 256) * -(-n_size // 256)) // w)
-    return (128, 512) if 1.6 * rounds_wide < rounds_square else (256, 256)
+    avg = max(-(-m_total // num_experts), 1)
+    rows = avg + 2 * math.isqrt(avg)
+
+    def rounds(tile_m, tile_n, r):
+        return -(-(num_experts * -(-r // tile_m) * -(-n_size // tile_n)) // w)
+
+    best, cost = (256, 256), math.inf
+    for tile, per_round in _TILE_ROUND_COST:
+        if tile == (128, 256) and rows <= 128:
+            per_round = 0.9
+        c = per_round * rounds(*tile, rows)
+        if c < cost:
+            best, cost = tile, c
+    if n_size >= 512 and avg <= 128 and 1.6 * rounds(128, 512, avg) < cost:
+        best = (128, 512)
+    return best
 
 
 def _requested_tile(block_m, block_n) -> Tuple[int, int]:

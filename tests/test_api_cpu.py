@@ -137,3 +137,16 @@ def test_odd_n_tiles():
     assert gg._odd_n_tile((192, 128), False) == (128, 128)
     for t in ((64, 64), (128, 64), (64, 128)):
         assert gg._odd_n_tile(t, True) == (128, 128)
+
+
+@pytest.mark.parametrize("rows,experts,n,want", [
+    (8 * 200, 8, 2048, (128, 128)),    # 64 square tiles: a quarter of the chip
+    (2222, 12, 2050, (256, 128)),      # 108: halves fill one round, quarters take two
+    (24 * 16, 24, 4096, (128, 128)),   # 1.5 rounds
+    (32 * 16, 32, 2048, (128, 256)),   # one full round of one m-tile each
+    (16 * 192, 16, 4096, (256, 256)),  # one full round
+    (16 * 1024, 16, 2048, (256, 256)),
+])
+def test_default_tile_fills_the_chip(rows, experts, n, want):
+    """Where 256x256 tiles leave CUs idle the default goes to smaller ones."""
+    assert gg._default_kernel_tile(rows, experts, n) == want
