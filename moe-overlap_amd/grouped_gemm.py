@@ -269,7 +269,7 @@ def _default_kernel_tile(m_total: int, num_experts: int, n_size: int = 4096,
     leaves the chip idle.  A round costs, in rounds of 256x256, 1.6 on 128x512
     (at most 128 rows an expert and N >= 512: it reads A half as often), 0.7 on
     256x128 and 128x256 and 0.5 on 128x128; with one m-tile an expert either
-    way, 128x256 streams the columns 256x256 does and costs 0.9.  Ties go to the larger tile.  Rows
+    way, 128x256 streams the columns 256x256 does and costs the same.  Ties go to the larger tile.  Rows
     per expert are taken two standard deviations above the average that top-k
     routing spreads them around, so that a tile edge just above the average is
     not counted on (128x512 goes by the average itself).
@@ -284,7 +284,9 @@ def _default_kernel_tile(m_total: int, num_experts: int, n_size: int = 4096,
     94.5 / 93.7, 81.1 / 80.7, 128x256 87.9 / 89.4; E=64 x 16 rows, K=1024,
     N=1408 (384) 54.8 / 55.1, 56.6 / 54.7, 45.3 / 44.1, 49.7 / 49.7.
     One m-tile an expert, a full round: E=32 x 16 rows, K=7168, N=2048 (256)
-    192.7 / 181.1 against 128x256 171.3 / 167.7.
+    192.7 / 181.1 against 128x256 171.3 / 167.7 by events, level (173.5 and
+    173.2) in a run of calls; E=40 x 40 rows skewed, K=448, N=4282, fp16,
+    [E, N, K] 25.4 against 28.4.
     Rounds full: E=16 x 192 rows, K=2048, N=4096 (256) 256x256 63.2 / 62.4
     against 128x256 101.2 / 98.5; 256-384 rows 101-119 against 140-192.
     128x512: E=256 x 128 rows, K=7168, N=2048 1271 against 1584 (256x256);
@@ -302,7 +304,7 @@ def _default_kernel_tile(m_total: int, num_experts: int, n_size: int = 4096,
     best, cost = (256, 256), math.inf
     for tile, per_round in _TILE_ROUND_COST:
         if tile == (128, 256) and rows <= 128:
-            per_round = 0.9
+            per_round = 1.0
         c = per_round * rounds(*tile, rows)
         if c < cost:
             best, cost = tile, c

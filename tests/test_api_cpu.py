@@ -143,7 +143,8 @@ def test_odd_n_tiles():
     (8 * 200, 8, 2048, (128, 128)),    # 64 square tiles: a quarter of the chip
     (2222, 12, 2050, (256, 128)),      # 108: halves fill one round, quarters take two
     (24 * 16, 24, 4096, (128, 128)),   # 1.5 rounds
-    (32 * 16, 32, 2048, (128, 256)),   # one full round of one m-tile each
+    (32 * 16, 32, 2048, (256, 256)),   # one full round of one m-tile each
+    (40 * 40, 40, 4282, (256, 256)),   # 3 rounds against 6 of a half each
     (16 * 192, 16, 4096, (256, 256)),  # one full round
     (16 * 1024, 16, 2048, (256, 256)),
 ])
