@@ -75,6 +75,26 @@ __device__ __forceinline__ P* uniform_ptr(P* ptr) {
   return reinterpret_cast<P*>(((uint64_t)hi << 32) | lo);
 }
 
+// dma16 with no scalar offset: the lane offset and the record count alone decide
+// what is read (whether the range check sees a scalar offset is not relied on).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16_at(i32x4 rsrc, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+               :
+               : "v"(voff), "s"(rsrc), "s"(lds)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// The descriptor `bytes` further on: its base moved, its records as many fewer
+// (none below none).
+__device__ __forceinline__ void advance_rsrc(i32x4& r, int bytes) {
+  const uint64_t base = (((uint64_t)(uint32_t)r[1] << 32) | (uint32_t)r[0]) + (uint64_t)bytes;
+  r[0] = (int32_t)(uint32_t)base;
+  r[1] = (int32_t)(uint32_t)(base >> 32);
+  r[2] = r[2] > bytes ? r[2] - bytes : 0;
+}
+
 template <class T, int EPI>
 __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles, int32_t w_report,
                                            int32_t first, int n_tiles, const int32_t* s_prefix,
@@ -198,8 +218,8 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
   // Chunk (row, K position) a lane moves in its wave's t-th A or B DMA of a
   // stage: 8 rows of 128 bytes each; chunk c of row r lies at
   // c ^ ((r >> 1) & 7).
-  i32x4 a_rsrc, b_rsrc;
-  int iss_k0 = 0;    // K position of the next stage to issue
+  i32x4 a_rsrc, b_rsrc;  // from the next stage to issue on
+  int iss_k0 = 0;    // K position of that stage
   int iss_klen = 0;  // K extent of the source tile (a part's, for a split tile)
   auto row_of = [&](int l, int t) { return 8 * (8 * wave + t) + (l >> 3); };
   auto kpos_of = [&](int l, int t) { return 8 * ((l & 7) ^ ((l >> 4) | (4 * (t & 1)))); };
@@ -248,11 +268,15 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
   };
   const uint32_t lds0 = lds_addr(lds);
   const uint32_t dst0 = lds0 + wave * 8192;
-  // DMA d (0-7 B, 8-15 A) of the stage at iss_k0 into the slot at byte `slot`.
+  // DMA d (0-7 B, 8-15 A) of the next stage into the slot at byte `slot`.
   auto issue = [&](uint32_t slot, int d) {
-    const uint32_t k_off = (uint32_t)iss_k0 * 2;
-    dma16(d < 8 ? b_rsrc : a_rsrc, d < 8 ? b_voff[d] : a_voff[d - 8],
-          __builtin_amdgcn_readfirstlane(k_off), dst0 + slot + (d < 8 ? 32768 : 0) + d % 8 * 1024);
+    dma16_at(d < 8 ? b_rsrc : a_rsrc, d < 8 ? b_voff[d] : a_voff[d - 8],
+             dst0 + slot + (d < 8 ? 32768 : 0) + d % 8 * 1024);
+  };
+  auto next_stage = [&]() {
+    iss_k0 += kKmStage;
+    advance_rsrc(a_rsrc, kKmStage * 2);
+    advance_rsrc(b_rsrc, kKmStage * 2);
   };
   auto no_source = [&]() {  // nothing left to load: every DMA writes zeros
     a_rsrc[2] = 0;
@@ -496,7 +520,7 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
     set_offsets(iss_klen - iss_k0);
 #pragma unroll
     for (int d = 0; d < 16; ++d) issue(s * kKmSlot, d);
-    iss_k0 += kKmStage;
+    next_stage();
   }
   wait_dma<16>();
   __syncthreads();
@@ -606,7 +630,7 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
         if (x % kDmaGap == 1 && kOut + x / kDmaGap < 16) issue(slot, kOut + x / kDmaGap);
         __builtin_amdgcn_sched_barrier(0);
       }
-      iss_k0 += kKmStage;
+      next_stage();
       slot = other;
     }
     if (s < ns) continue;
