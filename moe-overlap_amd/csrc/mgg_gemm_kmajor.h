@@ -352,27 +352,33 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
   // bytes a row, 16-byte chunk ch of row r at ch ^ r, conflict-free both
   // ways); each lane takes 8 consecutive columns back, applies the epilogue
   // and stores 16 bytes, 128 consecutive bytes of a row per 8 lanes (64 per 4
-  // with SwiGLU, whose 64 columns are 32 gates and their 32 ups).  Where the
-  // tile's columns all exist and C's rows are 16-byte aligned they go as
-  // buffer stores, rows that do not exist masked by offset, so that every such
-  // tile issues kStores of them and the next tile's first wait counts past
-  // them.
+  // with SwiGLU, whose 64 columns are 32 gates and their 32 ups).  Where C's
+  // rows are whole 16-byte chunks they go as buffer stores, rows and columns
+  // that do not exist masked by offset, so that every such tile issues kStores
+  // of them and the next tile's first wait counts past them.
   constexpr int kStores = kEpi == kEpiSwiglu ? 16 : 32;
   uint8_t* const rows_lds = s_rows + wave * kKmRow;
-  auto counted = [&](const Coords& c) {
+  auto counted = [&]() {
     const KernelArgs p = kernel_args();
     const int64_t c_cols = kEpi == kEpiSwiglu ? p->n / 2 : p->n;
-    const int64_t end = kEpi == kEpiSwiglu ? c.n0 / 2 + 128 : c.n0 + 256;
-    return end <= c_cols && (p->ldc & 7) == 0 && p->ldc < (1 << 21);
+    return ((c_cols | p->ldc) & 7) == 0 && p->ldc < (1 << 21);
   };
-  // MODE kOutBuffered: as above; kOutPlain: any other tile; kOutParts: the
-  // other parts' sums added; kOutPartial: a part's sums to its slot, as they
-  // come back from LDS (quad n of a lane at n * 4096 + wave * 1024 + 16 * lane).
-  constexpr int kOutBuffered = 0, kOutPlain = 1, kOutParts = 2, kOutPartial = 3;
-  auto epilogue = [&](auto Mode, const Coords& c) {
+  // kMode kOutBuffered: as above; kOutPlain: any other C; kOutPartial: a
+  // part's sums to its slot, as they come back from LDS (quad n of a lane at
+  // n * 4096 + wave * 1024 + 16 * lane).  kOthers: how many other parts' sums
+  // are added (3 also for two, the missing one reading as zeros).  They lie in
+  // uncached memory, microseconds away, so they are read kAhead of the 16
+  // steps ahead, as many as the registers hold without a spill (the plain
+  // stores' addresses leave room for none).  Read in their own step, the
+  // halves of 8 experts x 256 rows, K = 2048, N = 4096 took 65.2 us, now 50.5
+  // (whole tiles 62.1).
+  constexpr int kOutBuffered = 0, kOutPlain = 1, kOutPartial = 2;
+  auto epilogue = [&](auto Mode, auto Others, const Coords& c) {
     constexpr int kMode = decltype(Mode)::value;
+    constexpr int kOthers = decltype(Others)::value;
     constexpr bool kBuf = kMode == kOutBuffered;
-    constexpr bool kParts = kMode == kOutParts;
+    constexpr bool kParts = kOthers > 0;
+    constexpr int kAhead = !kBuf ? 0 : kOthers == 1 ? 4 : 1;
     constexpr int kLanes = kEpi == kEpiSwiglu ? 4 : 8;  // lanes to a row
     const KernelArgs p = kernel_args();
     const int64_t c_cols = kEpi == kEpiSwiglu ? p->n / 2 : p->n;
@@ -401,13 +407,29 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
       return *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(
           lds_ptr(rows_lds) + rr * 256 + ((cc ^ rr) * 16));
     };
-    auto summed = [&](f32x4 v, int at) -> f32x4 {
+    constexpr int kRing = kAhead > 0 ? kAhead : 1;
+    f32x4 others[kRing][kParts ? kOthers : 1][2][2];  // step n's at n % kRing
+    auto read_part = [&](auto r, int at) -> f32x4 {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, part_off, at, 17));
+    };
+    auto read_others = [&](int n) {
       if constexpr (kParts) {
-        const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r_pair, part_off, at, 17));
-        const f32x4 b0 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r_far0, part_off, at, 17));
-        const f32x4 b1 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r_far1, part_off, at, 17));
-        v = (v + a) + (b0 + b1);
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) {
+            const int at = quad_at(n, g, hh);
+            others[n % kRing][0][g][hh] = read_part(r_pair, at);
+            if constexpr (kOthers == 3) {
+              others[n % kRing][1][g][hh] = read_part(r_far0, at);
+              others[n % kRing][2][g][hh] = read_part(r_far1, at);
+            }
+          }
       }
+    };
+    auto summed = [&](f32x4 v, int n, int g, int hh) -> f32x4 {
+      if constexpr (kParts) v += others[n % kRing][0][g][hh];
+      if constexpr (kOthers == 3) v += others[n % kRing][1][g][hh] + others[n % kRing][2][g][hh];
       return v;
     };
     const auto r_own = __builtin_amdgcn_make_buffer_rsrc(
@@ -426,6 +448,11 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
     // step's are read back while the step before it is stored (LDS operations
     // of a wave run in order, so its writes need no wait for those reads).
     f32x4 back[2][2][2];
+    if constexpr (kParts) {
+#pragma unroll
+      for (int n = 0; n < kAhead; ++n) read_others(n);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int n = 0; n <= 16; ++n) {
       if (n < 16) {
@@ -453,11 +480,13 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) store_quad(back[(n - 1) & 1][g][hh], quad_at(n - 1, g, hh));
       } else {
+        if (kParts && kAhead == 0) read_others(n - 1);
         f32x4 v[2][2];
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
-          for (int hh = 0; hh < 2; ++hh) v[g][hh] = summed(back[(n - 1) & 1][g][hh], quad_at(n - 1, g, hh));
+          for (int hh = 0; hh < 2; ++hh) v[g][hh] = summed(back[(n - 1) & 1][g][hh], n - 1, g, hh);
+        if (kAhead > 0 && n - 1 + kAhead < 16) read_others(n - 1 + kAhead);
 #pragma unroll
         for (int u = 0; u < kLanes / 4; ++u) {
           float y[8];
@@ -470,7 +499,7 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
                            T::pack(y[6], y[7])};
           const int mr = wm * 128 + 16 * j + 64 / kLanes * u + l / kLanes;
           const int64_t col = col0 + h * (kEpi == kEpiSwiglu ? 32 : 64);
-          const bool ok = mr >= row_lo && mr < row_hi;
+          const bool ok = mr >= row_lo && mr < row_hi && col < c_cols;
           if constexpr (kBuf) {
             const uint32_t off = (uint32_t)((mr * (int32_t)p->ldc + (int32_t)col) * 2);
             __builtin_amdgcn_raw_buffer_store_b128(w, c_rsrc, ok ? (int)off : (int)kOutOfRange, 0, 2);
@@ -634,22 +663,27 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
       slot = other;
     }
     if (s < ns) continue;
-        if (cur.slot >= 0) {
+    if (cur.slot >= 0) {
       int last = same(others_done(cur) ? 1 : 0);
       if (last == 0) {
-        epilogue(IntConst<kOutPartial>{}, cur);
+        epilogue(IntConst<kOutPartial>{}, IntConst<0>{}, cur);
         last = same(last_to_write(cur) ? 1 : 0);
       }
       if (last != 0) {
         if (tid == 0)
           __hip_atomic_store(split_flag(kernel_args(), cur), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        epilogue(IntConst<kOutParts>{}, cur);
+        if (!counted())
+          epilogue(IntConst<kOutPlain>{}, IntConst<3>{}, cur);
+        else if (split_s == 2)
+          epilogue(IntConst<kOutBuffered>{}, IntConst<1>{}, cur);
+        else
+          epilogue(IntConst<kOutBuffered>{}, IntConst<3>{}, cur);
       }
-    } else if (counted(cur)) {
-      epilogue(IntConst<kOutBuffered>{}, cur);
+    } else if (counted()) {
+      epilogue(IntConst<kOutBuffered>{}, IntConst<0>{}, cur);
       stores_behind = 1;
     } else {
-      epilogue(IntConst<kOutPlain>{}, cur);
+      epilogue(IntConst<kOutPlain>{}, IntConst<0>{}, cur);
     }
     if (!more) break;
     cur = nxt;

@@ -5,6 +5,7 @@ same fp32 sum in the same K order)."""
 import pytest
 import torch
 
+import expert_mlp as mlp
 import grouped_gemm as gg
 from test_gpu_gemm import assert_parity, covered_rows, kmajor_copy, log, make_inputs
 
@@ -62,3 +63,74 @@ def test_kmajor_split_last_round(cuda_device, parts, workers):
         assert torch.equal(outs[0][: counts[0]], outs[1][: counts[0]])
         assert torch.equal(outs[0][: counts[0]], outs[2][: counts[0]])
         assert_parity(outs[0], a, b, offs, k)
+
+
+def _fused(a, b, offs, activation, block, workers, atomic):
+    out = b.shape[2] // 2 if activation == "swiglu" else b.shape[2]
+    return mlp._grouped_gemm_ex(a, b, offs, mlp._EPILOGUES[activation], out, workers, block, atomic)
+
+
+# N: whole tiles; a last tile whose columns end inside a wave's half; C's rows
+# not whole 16-byte chunks (GELU only: SwiGLU's N is a multiple of 64).
+@pytest.mark.parametrize("activation,n", [("gelu", 512), ("gelu", 320), ("gelu", 516), ("swiglu", 512),
+                                          ("swiglu", 320), ("swiglu", 704)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_kmajor_fused_epilogues(cuda_device, activation, n, dtype):
+    """The activations on several tiles a worker (the next tile's loads behind
+    the stores), several stages of K and a part of one: bitwise the 128x128
+    tile's."""
+    counts, k = [300, 0, 257, 1, 200], 1032
+    a, b, offs = make_inputs(counts, k, n, dtype, cuda_device, seed=n, extra_rows=1)
+    b_km = kmajor_copy(b, 16)
+    rows = sum(counts)
+    want = _fused(a, b_km, offs, activation, 128, None, False)
+    for atomic, workers in ((False, 2), (True, 3), (True, 1)):
+        log(f"kmajor fused {activation} n={n} {dtype} atomic={atomic} workers={workers}")
+        got = _fused(a, b_km, offs, activation, 256, workers, atomic)
+        torch.cuda.synchronize()
+        assert torch.equal(got[:rows], want[:rows]), (atomic, workers)
+
+
+@pytest.mark.parametrize("activation,n", [("none", 320), ("none", 516), ("gelu", 512), ("gelu", 516),
+                                          ("swiglu", 320)])
+@pytest.mark.parametrize("tiles,k", [(8, 2248), (5, 3272), (4, 4160)])  # halves, thirds, quarters of K
+def test_kmajor_split_epilogues(cuda_device, activation, n, tiles, k):
+    """Tiles summed in parts of K under every epilogue, with columns that do
+    not fill the tile.  The whole tile's sum and the parts' differ by fp32
+    rounding (about 1e-5 of unit-scale sums, at most 1e-4 after the
+    activation), so the bf16 results differ by a rounding at most."""
+    workers, counts = 16, [256 * (tiles // 2) - 5]
+    a, b, offs = make_inputs(counts, k, n, torch.bfloat16, cuda_device, seed=tiles, extra_rows=1)
+    b_km = kmajor_copy(b, 0)
+
+    def run(block, num_sms, atomic):
+        if activation == "none":
+            return gg.persistent_grouped_gemm(a, b_km, offs, kernel_tile=(block, block), num_sms=num_sms,
+                                              use_atomic_queue=atomic)[: counts[0]]
+        return _fused(a, b_km, offs, activation, block, num_sms, atomic)[: counts[0]]
+
+    log(f"kmajor split {activation} n={n} tiles={tiles} k={k}")
+    want = run(128, None, False)
+    outs = [run(256, workers, True) for _ in range(3)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    torch.testing.assert_close(outs[0].float(), want.float(), rtol=2.0 ** -7, atol=1e-4)
+
+
+@pytest.mark.parametrize("experts", [64, 65, 129, 1000, 2048])
+def test_kmajor_finds_the_expert(cuda_device, experts):
+    """Device-derived tiles of more experts than a wave has lanes, empty ones
+    among them, more than one m-tile in a few."""
+    gen = torch.Generator().manual_seed(experts)
+    counts = torch.randint(0, 6, (experts,), generator=gen)
+    counts[torch.randint(0, experts, (3,), generator=gen)] = 300
+    counts[-1] = 2
+    k, n = 72, 258
+    a, b, offs = make_inputs(counts.tolist(), k, n, torch.bfloat16, cuda_device, seed=experts)
+    b_km = kmajor_copy(b, 0)
+    want = gg.persistent_grouped_gemm(a, b_km, offs, kernel_tile=(128, 128), use_atomic_queue=False)
+    for atomic in (False, True):
+        log(f"kmajor experts={experts} atomic={atomic}")
+        got = gg.persistent_grouped_gemm(a, b_km, offs, kernel_tile=(256, 256), num_sms=3, use_atomic_queue=atomic)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), atomic
