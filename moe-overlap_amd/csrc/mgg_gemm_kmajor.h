@@ -16,19 +16,21 @@
 //           per kDmaGap MFMAs;
 //   wait for the next stage's DMAs, barrier;
 //   step 1: 64 MFMAs on set 1; the rest of the DMAs; set 0 of the next stage.
-// (One DMA per MFMA holds up the only wave of its SIMD: 1270 against 1377
-// TFLOP/s at a gap of 4 on a dense 16384 x 4096 x 8192 problem.)  The stage
+// (One DMA per MFMA holds up the only wave of its SIMD: 1323 TFLOP/s from
+// MFMA 47 on, 1475 from 35 on at a gap of 4, on a dense 16384 x 4096 x 8192
+// problem; a gap of 3 from 33 on is level there and 1-6% behind on the shapes
+// below.)  The stage
 // stream does not stop at a tile's end: its last two bodies issue the next
 // tile's stages 0 and 1, so they load behind the finished tile's epilogue, and
 // its stores drain behind the next tile's MFMAs.
 //
-// Measured against the eight-wave kernel it took the place of (ring of two
-// 64-deep stages, v_mfma_f32_32x32x16, one box, inputs in rotation): E = 16,
-// 1024 rows routed, K = 2048, N = 4096 302 -> 286 us; E = 8 x 2048 rows, N =
-// 8192 509 -> 464; E = 32, 300 rows, K = 1024, N = 2048 76.3 -> 68.3; one
-// m-tile per expert, where B streams from HBM (256 rows, K = 7168) 153.8 ->
-// 155.3.  The same kernel with N-major B (transposing reads) ran 3-6% behind
-// the eight-wave A-block kernel and is not built.
+// Measured against the eight-wave kernel (ring of two 64-deep stages,
+// v_mfma_f32_32x32x16), one process, inputs in rotation, atomic: E = 16, 1024
+// rows routed, K = 2048, N = 4096 297.7 -> 247.2 us; E = 8 x 2048 rows, N = 8192
+// 496.3 -> 429.5; E = 32, 300 rows, K = 1024, N = 2048 70.4 -> 60.2; one m-tile
+// per expert in halves of K (16 x 256 rows, K = 7168, N = 2048) 146.1 -> 125.1;
+// the dense problem 890.9 -> 745.3.  The same kernel with N-major B
+// (transposing reads) ran behind the eight-wave A-block kernel and is not built.
 #pragma once
 
 #include "mgg_gemm_kernel.h"
@@ -47,8 +49,7 @@ __device__ __forceinline__ f32x4 mfma16(F16, u32x4 a, u32x4 b, f32x4 c) {
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-// (35/4 and 35/6 within 1%, 47/4 4% slower on the shapes above.)
-constexpr int kFreeAt = 33, kDmaGap = 3;
+constexpr int kFreeAt = 35, kDmaGap = 4;
 constexpr int kKmThreads = 256;
 constexpr int kKmStage = 64;                 // K per stage
 constexpr int kKmSlot = 65536;               // LDS bytes of a stage: A, then B
@@ -639,6 +640,7 @@ __device__ __forceinline__ void run_kmajor(const GemmParams& p0, int32_t W_tiles
         __builtin_amdgcn_sched_barrier(0);
       }
       constexpr int kOut = (63 - kFreeAt) / kDmaGap;  // DMAs of this body so far
+      static_assert(kOut + (62 / kDmaGap + 1) >= 16, "a body issues a stage's sixteen DMAs");
       if (stores_behind != 0) {
         wait_dma<kStores + kOut>();
         stores_behind = 0;
