@@ -23,8 +23,9 @@ int launch_typed(int block_m, int block_n, const GemmParams& p, int workers, hip
   // rows) and as many stages as the LDS budget holds, except the 256x256
   // tile (see MGG_SBK256).  Fused epilogues are compiled for the 256x256 and
   // 128x128 tiles (two 32-column blocks per wave).
-  // K-major B's 256x256 tile is mgg_gemm_kmajor.h's.
-  if constexpr (!T::kBKMajor) { MGG_CASE(256, 256, MGG_SBK256, MGG_NS256, MGG_NW256) }
+  constexpr int kSbk256 = T::kBKMajor ? MGG_KM_SBK256 : MGG_SBK256;
+  constexpr int kNs256 = T::kBKMajor ? MGG_KM_NS256 : MGG_NS256;
+  MGG_CASE(256, 256, kSbk256, kNs256, MGG_NW256)
   MGG_CASE(128, 128, 64, 4, 4)
   if constexpr (EPI == kEpiNone) {
     MGG_CASE(256, 128, 64, 3, 4)
@@ -71,6 +72,19 @@ int launch_gathered(const GemmParams& p, int workers, hipStream_t stream) {
   return MGG_OK;
 }
 
+// Whether K-major B's 256x256 tiles run mgg_gemm_kmajor.h's four waves: not
+// where K is short and each worker has a tile or two, whose first loads and
+// last stores stand alone and go faster on eight waves.  Four waves against
+// eight: K = 512, 64 x 200 rows, N = 768 (less than a round) 1.06 (GELU 1.06,
+// SwiGLU 1.11), 16 x 768 rows, N = 2816 (2.4 rounds) 0.93 (1.03, 1.06); K =
+// 1024, 8 x 64 rows, N = 768 1.00 (1.02, 1.04), 64 x 200 rows, N = 1024 (one
+// round) 0.92 (0.99, 1.01); K = 1408, 8 x 100 rows, N = 2816 0.97 (1.00, 1.01).
+bool four_waves(int epilogue, const GemmParams& p, int workers) {
+  const int64_t tiles = (p.m + 255) / 256 * ((p.n + 255) / 256);  // at least, if every row is routed
+  if (epilogue == kEpiNone) return p.k >= 1024 || tiles >= 2 * (int64_t)workers;
+  return p.k >= 1408 || (p.k >= 1024 && tiles >= workers);
+}
+
 template <class T>
 int launch_epi(int epilogue, int block_m, int block_n, const GemmParams& p, int workers,
                hipStream_t stream) {
@@ -89,7 +103,7 @@ int launch_epi(int epilogue, int block_m, int block_n, const GemmParams& p, int 
     if (p.a_rows != nullptr) return set_error(MGG_ERR_UNSUPPORTED, "gathered A needs N-major 16-bit B");
   }
   if constexpr (T::kBKMajor) {
-    if (block_m == 256 && block_n == 256)
+    if (block_m == 256 && block_n == 256 && four_waves(epilogue, p, workers))
       return launch_kmajor_256(std::is_base_of_v<Bf16, T> ? MGG_DTYPE_BF16 | MGG_B_KMAJOR
                                                           : MGG_DTYPE_FP16 | MGG_B_KMAJOR,
                                epilogue, p, workers, stream);

@@ -29,7 +29,7 @@
 #define MGG_SBK256 32
 #define MGG_NS256 4
 #endif
-// K-major 16-bit B on the 256x256 tile (odd N; even N runs
+// K-major 16-bit B on the 256x256 tile (odd N and short K; the rest runs
 // mgg_gemm_kmajor.h): both operands' rows run along K, so
 // 64-deep stages (full 128-byte lines for both, a ring of two) measured as
 // fast as a ring of four 32-deep stages on uniform counts and 4-7% faster

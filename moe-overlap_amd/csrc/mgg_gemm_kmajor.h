@@ -1,6 +1,7 @@
 // The 256x256 tile of the grouped GEMM for K-major 16-bit B ([E, N, K], a
-// linear layer's weights) and even N.  (N-major B, the other tiles, odd N and
-// fp8 run mgg_gemm_kernel.h, whose queue, tickets and static rounds this
+// linear layer's weights) and even N, where K is long or tiles are many
+// (four_waves in mgg_gemm.hip).  (N-major B, the other tiles, odd N, fp8 and
+// short K run mgg_gemm_kernel.h, whose queue, tickets and static rounds this
 // kernel shares.)
 //
 // What bounds it: the matrix cores, at the clock that power leaves them, and

@@ -43,6 +43,24 @@ def test_kmajor_256_edges(cuda_device, case, dtype):
     assert_parity(c, a, b, offs, k)
 
 
+@pytest.mark.parametrize("case", range(len(CASES) + 1))
+def test_kmajor_256_one_worker(cuda_device, case):
+    """Every tile on one worker, its loads running on from tile to tile: short
+    K keeps the four-wave kernel there (two tiles a worker), and K of less
+    than a stage, too."""
+    counts, k, n = (CASES + [([1, 0, 3], 8, 258)])[case]
+    a, b, offs = make_inputs(counts, k, n, torch.bfloat16, cuda_device, seed=400 + case, extra_rows=3)
+    b_km = kmajor_copy(b, 0)
+    mask = torch.from_numpy(covered_rows(offs)).to(cuda_device)
+    want = gg.persistent_grouped_gemm(a, b_km, offs, kernel_tile=(128, 128), use_atomic_queue=False)
+    for queue, atomic in (("device", False), ("device", True), ("prebuilt", True)):
+        log(f"kmajor one worker case={case} queue={queue} atomic={atomic}")
+        c = gg.persistent_grouped_gemm(a, b_km, offs, kernel_tile=(256, 256), queue=queue,
+                                       use_atomic_queue=atomic, num_sms=1)
+        torch.cuda.synchronize()
+        assert torch.equal(c[: mask.numel()][mask], want[: mask.numel()][mask]), (queue, atomic)
+
+
 @pytest.mark.parametrize("parts,workers", [(2, 16), (3, 16), (4, 16)])
 def test_kmajor_split_last_round(cuda_device, parts, workers):
     """Tiles of a short last round summed as 2, 3 or 4 parts of K (at least
