@@ -379,11 +379,12 @@ int mgg_gather_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token
                     int64_t ld_out, void* stream);
 
 /*
- * mgg_gather_rows over a whole dispatch layout (num_tokens * top_k rows, of
- * x's first num_tokens rows), given both of its index arrays: slot_position
- * and token_index must be the two directions of one mapping, as
- * mgg_dispatch_layout writes them.  Same result; either array is used,
- * whichever moves fewer bytes.
+ * mgg_gather_rows over a whole dispatch layout (max_rows = num_tokens * top_k,
+ * < 2^31), given both of its index arrays: the same arguments are refused and
+ * the result is the same, out[p, :] = x[token_index[p], :] for p < *num_rows.
+ * x has at least num_tokens rows.  Where slot_position [num_tokens * top_k] is
+ * token_index's inverse, as mgg_dispatch_layout writes it, a token's row is
+ * read once for all of its slots; rows it does not name are copied one by one.
  */
 int mgg_permute_rows(int dtype, const void* x, int64_t ld_x, const int32_t* slot_position,
                      const int32_t* token_index, const int32_t* num_rows, int64_t num_tokens,

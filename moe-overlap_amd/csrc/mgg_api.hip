@@ -804,10 +804,9 @@ int mgg_dispatch_layout_noalloc(const void* topk_idx, int idx_type, int64_t num_
                              slot_position, token_index, row_assignment, ws, need, stream);
 }
 
-int mgg_gather_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token_index,
-                    const int32_t* num_rows, int64_t max_rows, int64_t hidden, void* out,
-                    int64_t ld_out, void* stream) {
-  mgg::clear_error();
+// The argument checks that mgg_gather_rows and mgg_permute_rows share.
+static int check_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token_index,
+                      int64_t max_rows, int64_t hidden, const void* out, int64_t ld_out) {
   if (dtype != MGG_DTYPE_BF16 && dtype != MGG_DTYPE_FP16)
     return set_error(MGG_ERR_UNSUPPORTED, "dtype must be MGG_DTYPE_BF16 or MGG_DTYPE_FP16");
   if (max_rows < 0 || hidden < 0) return set_error(MGG_ERR_INVALID, "sizes must be >= 0");
@@ -816,6 +815,15 @@ int mgg_gather_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token
     return set_error(MGG_ERR_INVALID, "leading dimensions smaller than the row length");
   if (x == nullptr || token_index == nullptr || out == nullptr)
     return set_error(MGG_ERR_INVALID, "null pointer");
+  return MGG_OK;
+}
+
+int mgg_gather_rows(int dtype, const void* x, int64_t ld_x, const int32_t* token_index,
+                    const int32_t* num_rows, int64_t max_rows, int64_t hidden, void* out,
+                    int64_t ld_out, void* stream) {
+  mgg::clear_error();
+  const int rc = check_rows(dtype, x, ld_x, token_index, max_rows, hidden, out, ld_out);
+  if (rc != MGG_OK || max_rows == 0 || hidden == 0) return rc;
   return mgg::launch_gather_rows(x, ld_x, token_index, num_rows, max_rows, hidden, 2, out, ld_out,
                                  static_cast<hipStream_t>(stream));
 }
@@ -825,14 +833,17 @@ int mgg_permute_rows(int dtype, const void* x, int64_t ld_x, const int32_t* slot
                      int top_k, int64_t hidden, void* out, int64_t ld_out, void* stream) {
   mgg::clear_error();
   if (num_tokens < 0 || top_k < 0) return set_error(MGG_ERR_INVALID, "sizes must be >= 0");
+  if (top_k > 0 && num_tokens > (((int64_t)1 << 31) - 1) / top_k)
+    return set_error(MGG_ERR_UNSUPPORTED, "num_tokens * top_k must be < 2^31");
   const int64_t max_rows = num_tokens * top_k;
-  // One slot a token: nothing is read twice, and the gather's writes are in order.
-  if (top_k > 1 && (dtype == MGG_DTYPE_BF16 || dtype == MGG_DTYPE_FP16) && max_rows > 0 &&
-      hidden > 0 && ld_x >= hidden && ld_out >= hidden && x != nullptr && slot_position != nullptr &&
-      out != nullptr && mgg::scatter_rows_supported(x, ld_x, hidden, 2, out, ld_out))
-    return mgg::launch_scatter_rows(x, ld_x, slot_position, num_tokens, top_k, max_rows, hidden, 2,
-                                    out, ld_out, static_cast<hipStream_t>(stream));
-  return mgg_gather_rows(dtype, x, ld_x, token_index, num_rows, max_rows, hidden, out, ld_out, stream);
+  const int rc = check_rows(dtype, x, ld_x, token_index, max_rows, hidden, out, ld_out);
+  if (rc != MGG_OK || max_rows == 0 || hidden == 0) return rc;
+  if (slot_position == nullptr) return set_error(MGG_ERR_INVALID, "null slot_position");
+  if (mgg::scatter_rows_supported(x, ld_x, top_k, hidden, 2, out, ld_out))
+    return mgg::launch_scatter_rows(x, ld_x, slot_position, token_index, num_rows, num_tokens, top_k,
+                                    hidden, 2, out, ld_out, static_cast<hipStream_t>(stream));
+  return mgg::launch_gather_rows(x, ld_x, token_index, num_rows, max_rows, hidden, 2, out, ld_out,
+                                 static_cast<hipStream_t>(stream));
 }
 
 int mgg_combine_rows(int dtype, const void* y, int64_t ld_y, const int32_t* slot_position,

@@ -127,13 +127,14 @@ int launch_dispatch_layout(const void* topk_idx, int idx_type, int64_t num_token
 int launch_gather_rows(const void* x, int64_t ld_x, const int32_t* token_index,
                        const int32_t* rows_ptr, int64_t rows_max, int64_t hidden, int elem_bytes,
                        void* out, int64_t ld_out, hipStream_t stream);
-// launch_gather_rows' rows by the inverse positions; for the rows and strides
-// that scatter_rows_supported takes.
-bool scatter_rows_supported(const void* x, int64_t ld_x, int64_t hidden, int elem_bytes,
+// launch_gather_rows' num_tokens * top_k rows by the inverse positions; for the
+// rows and strides that scatter_rows_supported takes.
+bool scatter_rows_supported(const void* x, int64_t ld_x, int top_k, int64_t hidden, int elem_bytes,
                             const void* out, int64_t ld_out);
-int launch_scatter_rows(const void* x, int64_t ld_x, const int32_t* slot_pos, int64_t num_tokens,
-                        int top_k, int64_t rows_max, int64_t hidden, int elem_bytes, void* out,
-                        int64_t ld_out, hipStream_t stream);
+int launch_scatter_rows(const void* x, int64_t ld_x, const int32_t* slot_pos,
+                        const int32_t* token_index, const int32_t* rows_ptr, int64_t num_tokens,
+                        int top_k, int64_t hidden, int elem_bytes, void* out, int64_t ld_out,
+                        hipStream_t stream);
 int launch_combine_rows(int dtype, const void* y, int64_t ld_y, const int32_t* slot_pos,
                         const float* weight, int64_t num_tokens, int top_k, int64_t hidden,
                         void* out, int64_t ld_out, hipStream_t stream);

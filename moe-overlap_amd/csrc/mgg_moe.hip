@@ -362,33 +362,70 @@ gather_rows_kernel(const uint8_t* x, int64_t ld_x, const int32_t* token_index,
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// out[slot_pos[t, j], :] = x[t, :] for the slots with a position in
-// [0, rows_max): the gather above by its inverse, so a token's row is read
-// once and written top_k times, where the gather reads it from the far caches
-// top_k times.  One 16-byte chunk of one token per thread (blockIdx.y: which
-// kRowThreads chunks of the row), so every row's stores are in flight at once.
-// Bound by the writes.  Measured (T = 4096, top-8, H = 7168, 470 MB written):
-// gather 140.3 us, this 93.9 us (one box, kernel trace); the non-temporal hint for
-// outputs past the last-level cache's reach (kStreamBytes).
+// The gather above by the inverse of token_index: token t's row is read once
+// and written to its slots' positions, where the gather reads it from the far
+// caches top_k times.  One 16-byte chunk of one token per thread (blockIdx.y:
+// which kRowThreads chunks of the row), so every row's stores are in flight at
+// once.  Bound by the writes.  The result is the gather's whatever slot_pos
+// holds: a slot writes row p < rows only where token_index[p] is its token, and
+// a row that no slot of its token names (a layout whose arrays were changed
+// one without the other) is copied by token_index.  Each wave checks both for
+// its token's slots and for the rows t * top_k .. + top_k - 1 with a lane per
+// slot and per (row, slot), beside the load of the row.  Measured (T = 4096,
+// top-8, H = 7168, 470 MB written): gather 140.3 us, this 95.0 (93.9 without the
+// checks; kernel traces); non-temporal stores for outputs past the last-level
+// cache's reach (kStreamBytes).
+constexpr int kMaxScatterSlots = 64;  // a wave's lanes
+
 template <bool NT>
 __global__ void __launch_bounds__(kRowThreads)
 scatter_rows_kernel(const uint8_t* x, int64_t ld_x_bytes, const int32_t* slot_pos,
-                    int64_t num_tokens, int32_t top_k, int64_t rows_max, int64_t chunks,
-                    uint8_t* out, int64_t ld_out_bytes) {
+                    const int32_t* token_index, const int32_t* rows_ptr, int64_t num_tokens,
+                    int32_t top_k, int64_t rows_max, int64_t chunks, uint8_t* out,
+                    int64_t ld_out_bytes) {
+  const int lane = threadIdx.x & 63;
   const int64_t c = (int64_t)blockIdx.y * kRowThreads + threadIdx.x;
-  if (c >= chunks) return;
+  if (c - lane >= chunks) return;  // the whole wave
+  const bool here = c < chunks;
+  const int64_t rows = rows_ptr != nullptr ? (int64_t)*rows_ptr : rows_max;
+  const int64_t n = rows < rows_max ? rows : rows_max;
+  auto load = [&](int64_t t) {
+    return here ? reinterpret_cast<const u32x4*>(x + t * ld_x_bytes)[c] : u32x4{0u, 0u, 0u, 0u};
+  };
+  auto store = [&](int64_t row, const u32x4& v) {
+    u32x4* dst = reinterpret_cast<u32x4*>(out + row * ld_out_bytes) + c;
+    if (!here) return;
+    if constexpr (NT)
+      __builtin_nontemporal_store(v, dst);
+    else
+      *dst = v;
+  };
+  const int at_once = 64 / top_k;  // rows checked in one step
+  const int jl = lane / top_k, il = lane - jl * top_k;
+  const uint64_t slots_mask = top_k < 64 ? (1ull << top_k) - 1ull : ~0ull;
   for (int64_t t = blockIdx.x; t < num_tokens; t += gridDim.x) {
-    const u32x4 v = reinterpret_cast<const u32x4*>(x + t * ld_x_bytes)[c];
-    const int32_t* pos_t = slot_pos + t * top_k;
-    for (int j = 0; j < top_k; ++j) {
-      const int64_t pos = pos_t[j];
-      if (pos < 0 || pos >= rows_max) continue;
-      u32x4* dst = reinterpret_cast<u32x4*>(out + pos * ld_out_bytes) + c;
-      if constexpr (NT)
-        __builtin_nontemporal_store(v, dst);
-      else
-        *dst = v;
+    const u32x4 v = load(t);
+    int32_t pos = -1;
+    bool own = false;
+    if (lane < top_k) {
+      pos = slot_pos[t * top_k + lane];
+      own = pos >= 0 && pos < n && token_index[pos] == t;
     }
+    for (int j0 = 0; j0 < top_k; j0 += at_once) {
+      const int64_t r = t * top_k + j0 + jl;
+      const bool there = jl < at_once && j0 + jl < top_k && r < n;
+      const int32_t from = there ? token_index[r] : -1;
+      const bool named = there && from >= 0 && from < num_tokens &&
+                         slot_pos[(int64_t)from * top_k + il] == r;
+      const uint64_t names = __ballot(named);
+      uint64_t stray = __ballot(there && il == 0 && ((names >> (jl * top_k)) & slots_mask) == 0);
+      for (; stray != 0; stray &= stray - 1) {
+        const int l = __builtin_ctzll(stray);
+        store(t * top_k + j0 + l / top_k, load(__builtin_amdgcn_readlane(from, l)));
+      }
+    }
+    for (uint64_t todo = __ballot(own); todo != 0; todo &= todo - 1)
+      store(__builtin_amdgcn_readlane(pos, __builtin_ctzll(todo)), v);
   }
 }
 
@@ -582,16 +619,17 @@ int launch_gather_rows(const void* x, int64_t ld_x, const int32_t* token_index,
   return MGG_OK;
 }
 
-int launch_scatter_rows(const void* x, int64_t ld_x, const int32_t* slot_pos, int64_t num_tokens,
-                        int top_k, int64_t rows_max, int64_t hidden, int elem_bytes, void* out,
-                        int64_t ld_out, hipStream_t stream) {
-  if (num_tokens <= 0 || top_k <= 0 || rows_max <= 0 || hidden <= 0) return MGG_OK;
+int launch_scatter_rows(const void* x, int64_t ld_x, const int32_t* slot_pos,
+                        const int32_t* token_index, const int32_t* rows_ptr, int64_t num_tokens,
+                        int top_k, int64_t hidden, int elem_bytes, void* out, int64_t ld_out,
+                        hipStream_t stream) {
+  const int64_t rows_max = num_tokens * top_k;
   const int64_t chunks = hidden * elem_bytes / 16;
   const dim3 grid((unsigned)grid_for(num_tokens), (unsigned)((chunks + kRowThreads - 1) / kRowThreads));
 #define MGG_SCATTER(NT_)                                                                        \
   hipLaunchKernelGGL(scatter_rows_kernel<NT_>, grid, dim3(kRowThreads), 0, stream,              \
-                     (const uint8_t*)x, ld_x * elem_bytes, slot_pos, num_tokens, top_k, rows_max, \
-                     chunks, (uint8_t*)out, ld_out * elem_bytes)
+                     (const uint8_t*)x, ld_x * elem_bytes, slot_pos, token_index, rows_ptr,     \
+                     num_tokens, top_k, rows_max, chunks, (uint8_t*)out, ld_out * elem_bytes)
   if (rows_max * hidden * elem_bytes > kStreamBytes) MGG_SCATTER(true); else MGG_SCATTER(false);
 #undef MGG_SCATTER
   if (hipError_t err = hipGetLastError(); err != hipSuccess)
@@ -599,10 +637,11 @@ int launch_scatter_rows(const void* x, int64_t ld_x, const int32_t* slot_pos, in
   return MGG_OK;
 }
 
-bool scatter_rows_supported(const void* x, int64_t ld_x, int64_t hidden, int elem_bytes,
+bool scatter_rows_supported(const void* x, int64_t ld_x, int top_k, int64_t hidden, int elem_bytes,
                             const void* out, int64_t ld_out) {
   const int64_t row_bytes = hidden * elem_bytes;
-  return row_bytes % 16 == 0 && (ld_x * elem_bytes) % 16 == 0 && (ld_out * elem_bytes) % 16 == 0 &&
+  // One slot a token: nothing is read twice, and the gather's writes are in order.
+  return top_k > 1 && top_k <= kMaxScatterSlots && row_bytes % 16 == 0 && (ld_x * elem_bytes) % 16 == 0 && (ld_out * elem_bytes) % 16 == 0 &&
          aligned16(x) && aligned16(out) && row_bytes / 16 <= 65535LL * kRowThreads;
 }
 

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import expert_mlp as mlp
+import mgg_native as nat
 
 pytestmark = pytest.mark.gpu
 
@@ -37,6 +38,37 @@ def test_permute_rows(cuda_device, tokens, experts, top_k, hidden, pad, masked):
     # A layout that holds one direction only goes by token_index.
     one_way = dataclasses.replace(lay, slot_position=None)
     assert torch.equal(mlp.permute_tokens(x, one_way)[:n], want)
+
+
+@pytest.mark.parametrize("tokens,top_k,hidden", [(50, 3, 2056), (130, 8, 64), (7, 64, 16), (9, 65, 16)])
+def test_permute_rows_follows_token_index(cuda_device, tokens, top_k, hidden):
+    """A layout whose arrays were changed one without the other: the rows are
+    those of token_index up to offsets[E], whatever slot_position holds, and
+    rows past offsets[E] stay as they were."""
+    gen = torch.Generator().manual_seed(top_k)
+    lay = mlp.dispatch_layout(_routing(tokens, 2 * top_k, top_k, 0.2, cuda_device), 2 * top_k)
+    n, total = int(lay.offsets[-1]), lay.max_rows
+    x = torch.randn(tokens + 5, hidden, device=cuda_device).to(torch.float16)
+    slots = lay.slot_position
+    fewer = lay.offsets.clone()
+    fewer[-1] = n // 2
+    moved = lay.token_index.clone()  # other tokens' rows, among them rows past the layout's tokens
+    moved[:n] = torch.randint(0, tokens + 5, (n,), generator=gen).to(moved)
+    some = torch.where(torch.rand(total, generator=gen).to(cuda_device) < 0.3, -1, slots).to(torch.int32)
+    junk = torch.randint(-3, total + 3, (total,), generator=gen, dtype=torch.int32).to(cuda_device)
+    for what, changed in (("fewer rows", dict(offsets=fewer)), ("tokens moved", dict(token_index=moved)),
+                          ("slots dropped", dict(slot_position=some)), ("slots junk", dict(slot_position=junk)),
+                          ("both", dict(token_index=moved, slot_position=junk))):
+        changed = dataclasses.replace(lay, **changed)
+        rows = int(changed.offsets[-1])
+        want = x[changed.token_index[:rows].long()]
+        out = torch.full((total, hidden), 7.0, device=cuda_device, dtype=x.dtype)
+        nat.check(nat.lib().mgg_permute_rows(
+            nat.MGG_DTYPE_FP16, x.data_ptr(), hidden, changed.slot_position.data_ptr(),
+            changed.token_index.data_ptr(), changed.offsets[-1:].data_ptr(), tokens, top_k, hidden,
+            out.data_ptr(), hidden, torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(mlp.permute_tokens(x, changed)[:rows], want), what
+        assert torch.equal(out[:rows], want) and bool((out[rows:] == 7.0).all()), what
 
 
 @pytest.mark.parametrize("tokens,top_k,experts", [

@@ -179,3 +179,34 @@ def test_builders_validate():
         == nat.MGG_ERR_INVALID
     assert lib.mgg_expert_offsets_from_counts(FAKE, 5, 4, FAKE, 0, None) == nat.MGG_ERR_INVALID
     assert lib.mgg_expert_offsets_from_counts(None, 0, 4, FAKE, 0, None) == nat.MGG_ERR_INVALID
+
+
+def permute_call(**over):
+    args = dict(dtype=nat.MGG_DTYPE_BF16, x=FAKE, ld_x=64, slot=FAKE, tok=FAKE, rows=FAKE, tokens=4,
+                top_k=2, hidden=64, out=FAKE, ld_out=64, stream=None)
+    args.update(over)
+    return nat.lib().mgg_permute_rows(*args.values())
+
+
+@pytest.mark.parametrize("hidden", [64, 4])  # rows of whole 16-byte chunks and not
+@pytest.mark.parametrize("over, code, text", [
+    (dict(dtype=nat.MGG_DTYPE_FP8_E4M3), nat.MGG_ERR_UNSUPPORTED, b"dtype"),
+    (dict(x=None), nat.MGG_ERR_INVALID, b"null"),
+    (dict(tok=None), nat.MGG_ERR_INVALID, b"null"),
+    (dict(slot=None), nat.MGG_ERR_INVALID, b"null"),
+    (dict(out=None), nat.MGG_ERR_INVALID, b"null"),
+    (dict(ld_x=2), nat.MGG_ERR_INVALID, b"leading"),
+    (dict(ld_out=2), nat.MGG_ERR_INVALID, b"leading"),
+    (dict(tokens=-1), nat.MGG_ERR_INVALID, b">= 0"),
+    (dict(top_k=-1), nat.MGG_ERR_INVALID, b">= 0"),
+    (dict(tokens=1 << 30, top_k=2), nat.MGG_ERR_UNSUPPORTED, b"2^31"),
+    (dict(tokens=1 << 62, top_k=4), nat.MGG_ERR_UNSUPPORTED, b"2^31"),
+    (dict(tokens=0, x=None), nat.MGG_OK, b""),
+    (dict(top_k=0, x=None), nat.MGG_OK, b""),
+])
+def test_permute_rows_refuses_alike_on_both_paths(hidden, over, code, text):
+    """Whichever way the rows would move, the same calls are refused, before a
+    launch; negative row lengths as well."""
+    assert permute_call(hidden=hidden, **over) == code
+    assert text in nat.lib().mgg_last_error()
+    assert permute_call(hidden=-hidden) == nat.MGG_ERR_INVALID
