@@ -202,6 +202,18 @@ int mgg_grouped_gemm(int dtype, const void* a, const void* b, void* c,
                      int report_block_m, int report_block_n, void* stream);
 
 /*
+ * The tile (block_m << 16 | block_n) expected to be the fastest for
+ * mgg_grouped_gemm without a fused epilogue, from the sizes alone: dtype as
+ * there (BF16/FP16, optionally | MGG_B_KMAJOR; 0 for others), m_size rows over
+ * num_experts experts, num_workers workgroups; splits non-zero for the atomic
+ * schedule with the queue derived on the device (its last round may go in
+ * parts of K).  Every tile gives the same results to within fp32 summation
+ * order.
+ */
+int mgg_default_tile(int dtype, int64_t m_size, int64_t k_size, int64_t n_size, int64_t num_experts,
+                     int num_workers, int splits);
+
+/*
  * mgg_grouped_gemm with a fused element-wise epilogue.  Same arguments and
  * semantics otherwise (the queue is derived on the device when num_work < 0,
  * or read from work_expert/work_tile_m/work_tile_n, e.g. above 2048 experts).

@@ -4,6 +4,7 @@
 // message for mgg_last_error().
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <deque>
 #include <map>
 #include <mutex>
@@ -344,7 +345,113 @@ void clear_error() { g_last_error.clear(); }
 
 using mgg::set_error;
 
+namespace mgg {
+namespace {
+
+// The 16-bit kernel tile whose rounds of `workers` tiles cost least, from the
+// average rows per expert.  A round costs 1 on 256x256 and the shares below on
+// the others (fixed by measurement, a layout at a time: K-major B has another
+// 256x256 kernel; apart where an expert and its spread fit 128 rows, so that a
+// tile streams its columns of B and little else).  Rows past an expert's end
+// read nothing, so what decides is how far the last round leaves the chip idle.
+// Rounds are taken at two standard deviations above the average, around which
+// routed counts spread; where every expert can hold exactly the average (experts
+// divides m), half at that and half there: the call cannot see which it has (no
+// host sync on the offsets).  `splits` (atomic, queue derived on the device): a
+// last round that goes in 2-4 parts of K costs that share and the parts' meeting,
+// as long as kMeetingK of K.  Another tile has to win by kMargin, which the
+// spread of skewed counts eats first.  128x512 (N >= 512, at most 128 rows: it
+// reads A half as often) goes by the average alone.  Odd N has 256x256, 128x128
+// and, N-major, 128x512.
+//
+// Fitted on 360 problems (E 4-256, 1-1024 rows, K 512-7168, N 511-7168, uniform,
+// routed and skewed, both schedules); on 210 others the tile chosen takes 0.80
+// (N-major) and 0.76 (K-major) of 256x256's time on average and 4.1% and 2.0% more
+// than the best of the five, most where the routing is skewed.  Both sides of the lines (us, atomic / striped):
+//   8 x 256 rows, K = 2048, N = 4096 (half the chip at the average, all of it
+//   two deviations above): 256x256 50.3 / 57.9, 256x128 42.2 / 39.8, 128x128 52.6
+//   / 51.2; K-major 50.5 / 62.1, 45.4 / 43.3, 53.3 / 50.9;
+//   32 x 16 rows, K = 7168, N = 2048 (one round or two halves): N-major level
+//   (256x256 171.7 / 167.0, 128x128 169.6 / 168.4), K-major 183.8 / 180.3 against
+//   160.4 / 160.3 and 128x256 163.1 / 160.9;
+//   8 x 200 rows, K = 1024, N = 2048 (a quarter of the chip): 36.2 / 35.6, 128x128
+//   20.0 / 18.4;
+//   4 x 768 rows, K = 7168, N = 1408: 256x256 in thirds 83.7, 128x128 92.9, 256x128
+//   104.9 (it does not split there); in quarters, 16 x 160 rows, K = 4096, N =
+//   1024, 54.4 against 128x128, a whole round, 37.5;
+//   256 x 128 rows, K = 7168, N = 2048: N-major 128x512 1150 / 1162, 256x256 1568 /
+//   1558; K-major 1418 / 1420, 1597 / 1598 (routed 1770 against 1604).
+struct TileCosts {
+  double c256x128, c128x256, c128x128;
+};
+constexpr TileCosts kMany[2] = {{0.62, 0.90, 0.45}, {0.61, 0.75, 0.44}};  // [K-major]
+constexpr TileCosts kFew[2] = {{1.00, 0.95, 0.52}, {0.80, 0.78, 0.45}};
+constexpr double kMeetingK = 1638;
+constexpr double kWide[2] = {1.6, 1.8};
+constexpr double kMargin = 0.94;
+
+struct Tile {
+  int m, n;
+};
+
+Tile default_tile(bool kmajor, int64_t m, int64_t k, int64_t n, int64_t experts, int64_t workers,
+                  bool splits) {
+  constexpr Tile kSquare{256, 256};
+  if (experts <= 0 || n <= 0) return kSquare;
+  if (workers < 1) workers = 1;
+  const int64_t avg = std::max<int64_t>((m + experts - 1) / experts, 1);
+  const int64_t spread = avg + 2 * (int64_t)std::sqrt((double)avg);
+  auto rounds = [&](Tile t, int64_t rows) -> double {
+    const int64_t tiles = experts * ((rows + t.m - 1) / t.m) * ((n + t.n - 1) / t.n);
+    const int64_t whole = tiles / workers, rem = tiles % workers;
+    if (rem == 0) return (double)whole;
+    if (splits)
+      for (int s = 4; s >= 2; --s)
+        if (rem * s <= workers && k > 1024 * s - 64)
+          return whole + std::min(1.0, 1.0 / s + kMeetingK / (double)k);
+    return whole + 1.0;
+  };
+  const int64_t least_rows = m % experts == 0 ? avg : spread;
+  auto cost = [&](Tile t, double share) {
+    return share * 0.5 * (rounds(t, least_rows) + rounds(t, spread));
+  };
+  const TileCosts& c = spread <= 128 ? kFew[kmajor] : kMany[kmajor];
+  const bool odd = (n & 1) != 0;
+  const double square = cost(kSquare, 1.0);
+  Tile best = kSquare;
+  double least = kMargin * square;
+  const std::pair<Tile, double> others[] = {
+      {{256, 128}, c.c256x128}, {{128, 256}, c.c128x256}, {{128, 128}, c.c128x128}};
+  for (const auto& [t, share] : others) {
+    if (odd && t.m != t.n) continue;
+    const double v = cost(t, share);
+    if (v < least) {
+      best = t;
+      least = v;
+    }
+  }
+  constexpr Tile kWideTile{128, 512};
+  if (n >= 512 && avg <= 128 && !(odd && kmajor) &&
+      kWide[kmajor] * rounds(kWideTile, avg) < std::min(least, square))
+    best = kWideTile;
+  return best;
+}
+
+}  // namespace
+}  // namespace mgg
+
 extern "C" {
+
+int mgg_default_tile(int dtype, int64_t m_size, int64_t k_size, int64_t n_size, int64_t num_experts,
+                     int num_workers, int splits) {
+  const int base = dtype & ~MGG_B_KMAJOR;
+  if ((base != MGG_DTYPE_BF16 && base != MGG_DTYPE_FP16) || m_size < 0 || k_size < 0 || n_size < 0 ||
+      num_experts < 0)
+    return 0;
+  const mgg::Tile t = mgg::default_tile((dtype & MGG_B_KMAJOR) != 0, m_size, k_size, n_size,
+                                        num_experts, num_workers, splits != 0);
+  return t.m << 16 | t.n;
+}
 
 int mgg_abi_version(void) { return 8; }
 

@@ -8,12 +8,12 @@ The reference runs its experts as (src/train_moe_baseline.py:212-248, :335-341):
     out += y * gate                     (once per top-k slot)
 
 Here all T*k assignments go through in one pass, with no host
-synchronisation: the dispatch layout (two kernels, one up to 1024 assignments), the up-projection GEMM
-reading its rows through the layout (the row gather fused; a separate gather
-launch for shapes the fused path does not take) with the activation fused
-into its epilogue, the down-projection GEMM and the gate-weighted combine:
-five launches (four) on the current stream.  Buffers are
-sized for T*k rows; the kernels read the number of valid rows (offsets[E])
+synchronisation: the dispatch layout (two kernels; one up to 1024
+assignments), the up-projection GEMM reading its rows through the layout (the
+row gather fused; a separate launch for shapes the fused path does not take)
+with the activation fused into its epilogue, the down-projection GEMM and the
+gate-weighted combine: five launches (four) on the current stream.  Buffers
+are sized for T*k rows; the kernels read the number of valid rows (offsets[E])
 on the device.  Every op runs in libmgg.so (include/mgg.h); there is no
 fallback implementation.
 """
@@ -243,10 +243,11 @@ def _grouped_gemm_gathered(x, layout, w1, epilogue, out_cols, num_sms, use_atomi
 
 def _grouped_gemm_ex(a, b, offsets, epilogue, out_cols, num_sms, block, use_atomic_queue):
     """C [M, out_cols] = epilogue(A @ B[e]) over the expert row ranges, on the
-    block x block kernel tile (without an epilogue and block 256: on the GEMM's
-    own choice, smaller where that tile leaves CUs idle; the down projection of
-    32 tokens, top-2, 16 experts, F = 4096, H = 2048: 65 -> 55 us) (queue derived on the device; above 2048
-    experts prebuilt, as the drop-in does)."""
+    block x block kernel tile with the queue derived on the device (above 2048
+    experts prebuilt, as the drop-in does).  Without an epilogue block 256 means
+    the GEMM's own choice, smaller where that tile leaves CUs idle: the down
+    projection of 32 tokens, top-2, 16 experts, F = 4096, H = 2048 takes 55 us
+    so and 65 on 256x256."""
     if epilogue == nat.MGG_EPI_NONE:
         return persistent_grouped_gemm(a, b, offsets, num_sms=num_sms, block_m=block,
                                        block_n=block, use_atomic_queue=use_atomic_queue,

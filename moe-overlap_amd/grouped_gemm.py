@@ -21,8 +21,10 @@ Differences, all in arguments that do not change results:
   compiled tile, 256 x 256 for bf16/fp16 where its tiles fill the chip (eight
   waves, two per SIMD, 32-deep B stages and 64-deep A blocks) and smaller ones
   where they leave CUs idle, or the tile named by the keyword-only
-  ``kernel_tile``.  Every output element is the same fp32 sum in the same K
-  order whatever the tile, so results do not depend on either choice.
+  ``kernel_tile``.  Every output element of a whole tile is the same fp32 sum in
+  the same K order whatever the tile; the atomic schedule sums the tiles of a
+  short last round in 2-4 parts of K, so with it which outputs are summed in
+  parts depends on the tile (fp32 rounding; the striped schedule never does).
 * ``block_k``, ``num_warps``, ``num_stages`` are accepted and ignored: the
   kernel's K staging, wave count and LDS ring are fixed by its design.
 * ``queue="device"`` (default) derives the same (expert, tile_m, tile_n)
@@ -58,7 +60,6 @@ Differences, all in arguments that do not change results:
 from __future__ import annotations
 
 import ctypes
-import math
 import operator
 from typing import List, Optional, Tuple, Union
 
@@ -255,62 +256,16 @@ def _build_work_queue(
 # --------------------------------------------------------------------------
 # grouped GEMM
 # --------------------------------------------------------------------------
-# What a round of one tile per CU costs on each kernel tile, in rounds of
-# 256x256 (see _default_kernel_tile).
-_TILE_ROUND_COST = (((256, 256), 1.0), ((256, 128), 0.7), ((128, 256), 0.7), ((128, 128), 0.5))
-
-
-def _default_kernel_tile(m_total: int, num_experts: int, n_size: int = 4096,
-                         workers: int = 256) -> Tuple[int, int]:
-    """The tile whose rounds of `workers` tiles cost least, from the average
-    rows per expert (no host sync on the offsets).  Rows of a tile past its
-    expert's end are zero-fill DMAs that read nothing, so a tile's cost follows
-    its valid rows and its columns; what decides is how far the last round
-    leaves the chip idle.  A round costs, in rounds of 256x256, 1.6 on 128x512
-    (at most 128 rows an expert and N >= 512: it reads A half as often), 0.7 on
-    256x128 and 128x256 and 0.5 on 128x128; with one m-tile an expert either
-    way, 128x256 streams the columns 256x256 does and costs the same.  Ties go to the larger tile.  Rows
-    per expert are taken two standard deviations above the average that top-k
-    routing spreads them around, so that a tile edge just above the average is
-    not counted on (128x512 goes by the average itself).
-    Measured on MI355X (HIP-event medians of the call, atomic / striped, µs).
-    Fewer 256x256 tiles than workers: E=8 x 200 rows, K=1024, N=2048 (64
-    tiles) 256x256 36.2 / 35.6, 256x128 25.3 / 24.2, 128x128 20.0 / 18.4; the
-    same at K=7168 95.7 / 174.7, 81.2 / 103.0, 78.4 / 77.1; B as [E, N, K],
-    K=2048 60.5 / 62.8, 38.3 / 36.5, 29.4 / 28.1; E=12, 2222 rows, K=1504,
-    N=2050, fp16 (108 tiles) 48.1 / 47.7, 35.3 / 33.4, 45.9 / 43.5; E=16 x 4
-    rows, K=4096, N=2048 (128) 63.4 / 85.1, 57.9 / 59.8, 55.4 / 53.9.
-    A second round begun: E=24 x 16 rows, K=2048, N=4096 (384) 97.6 / 95.7,
-    94.5 / 93.7, 81.1 / 80.7, 128x256 87.9 / 89.4; E=64 x 16 rows, K=1024,
-    N=1408 (384) 54.8 / 55.1, 56.6 / 54.7, 45.3 / 44.1, 49.7 / 49.7.
-    One m-tile an expert, a full round: E=32 x 16 rows, K=7168, N=2048 (256)
-    192.7 / 181.1 against 128x256 171.3 / 167.7 by events, level (173.5 and
-    173.2) in a run of calls; E=40 x 40 rows skewed, K=448, N=4282, fp16,
-    [E, N, K] 25.4 against 28.4.
-    Rounds full: E=16 x 192 rows, K=2048, N=4096 (256) 256x256 63.2 / 62.4
-    against 128x256 101.2 / 98.5; 256-384 rows 101-119 against 140-192.
-    128x512: E=256 x 128 rows, K=7168, N=2048 1271 against 1584 (256x256);
-    E=128 x 32 rows, K=N=4096, 682 against 776; E=64 x 128, N=1024, 80.6
-    against 60.9."""
-    if num_experts <= 0:
-        return 256, 256
-    w = max(int(workers), 1)
-    avg = max(-(-m_total // num_experts), 1)
-    rows = avg + 2 * math.isqrt(avg)
-
-    def rounds(tile_m, tile_n, r):
-        return -(-(num_experts * -(-r // tile_m) * -(-n_size // tile_n)) // w)
-
-    best, cost = (256, 256), math.inf
-    for tile, per_round in _TILE_ROUND_COST:
-        if tile == (128, 256) and rows <= 128:
-            per_round = 1.0
-        c = per_round * rounds(*tile, rows)
-        if c < cost:
-            best, cost = tile, c
-    if n_size >= 512 and avg <= 128 and 1.6 * rounds(128, 512, avg) < cost:
-        best = (128, 512)
-    return best
+def _default_kernel_tile(m_total: int, num_experts: int, n_size: int = 4096, workers: int = 256,
+                         k_size: int = 1024, kmajor: bool = False, splits: bool = False) -> Tuple[int, int]:
+    """The 16-bit kernel tile whose rounds of `workers` tiles cost least, from
+    the sizes alone (the library's rule, where its reasons stand: 256x256 where
+    its tiles fill the chip, smaller ones where they leave CUs idle, 128x512 for
+    many experts of at most 128 rows).  `splits`: the atomic schedule with the
+    queue derived on the device, whose last round may go in parts of K."""
+    tile = _nat.lib().mgg_default_tile(_nat.MGG_DTYPE_BF16 | (_nat.MGG_B_KMAJOR if kmajor else 0),
+                                       m_total, k_size, n_size, num_experts, workers, splits)
+    return tile >> 16, tile & 0xFFFF
 
 
 def _requested_tile(block_m, block_n) -> Tuple[int, int]:
@@ -353,8 +308,8 @@ def _kmajor_layout(b: torch.Tensor) -> bool:
 def _odd_n_tile(tile: Tuple[int, int], wide_ok: bool) -> Tuple[int, int]:
     """Odd N runs on kernel instances of its own, compiled for 256x256 and
     128x128 tiles (and 128x512 when `wide_ok`: N-major 16-bit B): another
-    kernel tile computes on the nearest of these (the requested tile still
-    sets the queue the work_counter counts)."""
+    kernel tile named by the caller computes on the nearest of these (the
+    requested tile still sets the queue the work_counter counts)."""
     if tile in ((256, 256), (128, 128)) or (wide_ok and tile == (128, 512)):
         return tile
     return (256, 256) if max(tile) >= 256 else (128, 128)
@@ -443,11 +398,10 @@ def persistent_grouped_gemm(
         num_sms = _cu_count(dev_index)
     if int(num_sms) <= 0:
         raise ValueError("num_sms must be positive.")
-    if kernel_tile is None:
-        kernel_tile = _default_kernel_tile(m_total, num_experts, n_size, int(num_sms))
-    kbm, kbn = (int(v) for v in kernel_tile)
-    if (kbm, kbn) not in _KERNEL_TILES:
-        raise ValueError(f"kernel_tile must be one of {_KERNEL_TILES}.")
+    if kernel_tile is not None:
+        kbm, kbn = (int(v) for v in kernel_tile)
+        if (kbm, kbn) not in _KERNEL_TILES:
+            raise ValueError(f"kernel_tile must be one of {_KERNEL_TILES}.")
     counter_dev = _counter_arg(work_counter, use_atomic_queue, device)
 
     # K not a multiple of 8: A is zero-padded on the device to the next
@@ -458,7 +412,10 @@ def persistent_grouped_gemm(
     a_op, b_op = a_cat, b_expert
     # B stored [E, N, K] is read as it lies (no transposing copy).
     b_kmajor = k_pad == k_size and _kmajor_layout(b_expert)
-    if n_size & 1:
+    if kernel_tile is None:
+        kbm, kbn = _default_kernel_tile(m_total, num_experts, n_size, int(num_sms), k_size, b_kmajor,
+                                        bool(use_atomic_queue) and queue == "device")
+    elif n_size & 1:
         kbm, kbn = _odd_n_tile((kbm, kbn), not b_kmajor)
     if k_pad != k_size:
         a_op = torch.nn.functional.pad(a_op, (0, k_pad - k_size))

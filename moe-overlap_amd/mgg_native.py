@@ -112,7 +112,10 @@ _SIGNATURES = {
     ],
 }
 # entry points whose return value is not a status code
-_RESTYPES = {"mgg_dispatch_layout_workspace_bytes": ([_c_i64, _c_i32, _c_i64], _c_i64)}
+_RESTYPES = {
+    "mgg_dispatch_layout_workspace_bytes": ([_c_i64, _c_i32, _c_i64], _c_i64),
+    "mgg_default_tile": ([_c_i32, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32], _c_i32),
+}
 EXPORTED = tuple(_SIGNATURES) + tuple(_RESTYPES) + ("mgg_last_error",)
 
 _lib = None

@@ -151,3 +151,41 @@ def test_odd_n_tiles():
 def test_default_tile_fills_the_chip(rows, experts, n, want):
     """Where 256x256 tiles leave CUs idle the default goes to smaller ones."""
     assert gg._default_kernel_tile(rows, experts, n) == want
+
+
+@pytest.mark.parametrize("rows,experts,n,k,kmajor,splits,want", [
+    # K-major B has another 256x256 kernel: one round of few rows goes narrower.
+    (32 * 16, 32, 2048, 7168, False, False, (256, 256)),
+    (32 * 16, 32, 2048, 7168, True, False, (128, 256)),
+    # Counts that can all be equal: exact multiples of the tile are not counted up.
+    (8 * 256, 8, 4096, 2048, False, False, (256, 128)),
+    (8 * 256, 8, 4096, 2048, True, True, (256, 128)),
+    (16 * 512, 16, 1024, 2048, False, False, (256, 128)),
+    (8 * 256 - 1, 8, 4096, 2048, False, False, (256, 256)),  # cannot be equal
+    # Odd N: chosen among its own tiles.
+    (2222, 12, 2051, 1504, False, False, (128, 128)),
+    (18224, 68, 325, 2048, False, False, (128, 128)),
+    (64 * 8, 64, 4095, 7168, True, False, (128, 128)),  # no 128x512 with K-major B
+    # A last round in thirds or quarters of K (and K too short for them).
+    (4 * 768, 4, 1408, 7168, False, True, (256, 256)),
+    (4 * 768, 4, 1408, 7168, False, False, (256, 128)),
+    (4 * 768, 4, 1408, 2048, False, True, (256, 128)),
+    (16 * 160, 16, 1024, 4096, False, True, (128, 128)),
+    (0, 4, 64, 64, False, False, (128, 128)),
+    (5, 0, 64, 64, True, True, (256, 256)),
+])
+def test_default_tile_by_layout_and_counts(rows, experts, n, k, kmajor, splits, want):
+    assert gg._default_kernel_tile(rows, experts, n, 256, k, kmajor, splits) == want
+
+
+def test_default_tile_is_compiled_for_the_call():
+    """Every choice is a tile that the layout and N have kernels for."""
+    for experts in (1, 3, 16, 100, 3000):
+        for rows in (0, 1, 17, 4095, 30000):
+            for n in (1, 7, 64, 511, 513, 2048, 7169):
+                for kmajor in (False, True):
+                    for splits in (False, True):
+                        tile = gg._default_kernel_tile(rows, experts, n, 256, 4096, kmajor, splits)
+                        assert tile in gg._KERNEL_TILES
+                        if n & 1:
+                            assert tile == gg._odd_n_tile(tile, not kmajor)
