@@ -1,5 +1,6 @@
 """CPU model of the atomic schedule's split last round (the meeting protocol of
-split_fixup in moe-overlap_amd/csrc/mgg_gemm_kernel.h), run over random
+split_fixup in moe-overlap_amd/csrc/mgg_gemm_kernel.h, and at the end that of
+the K-major 256x256 kernel, which meets on one flag), run over random
 interleavings of the parts.
 
 The kernel's part q of split tile t (s parts, any s >= 2) meets its siblings in
@@ -110,3 +111,56 @@ def test_k_parts_cover_k(s, gran):
             assert abs(gq - want) <= 2 * gran, (k, q, gq, want)
         assert ends[0][0] == 0 and ends[-1][1] == k
         assert all(ends[i][1] == ends[i + 1][0] for i in range(s - 1))
+
+
+def run_tile_one_flag(s, t, flags, slots, stored):
+    """The meeting of the K-major 256x256 kernel (others_done, last_to_write in
+    moe-overlap_amd/csrc/mgg_gemm_kmajor.h): the s parts share flag word
+    (s-1)*t.  A part that finds s - 1 others done is the last and writes
+    nothing; any other writes its sums to slot s*t + q and takes a ticket, and
+    is the last if it draws s - 1.  The last returns the flag and adds the other
+    slots in the order (p0 + p1) + (p2 + p3)."""
+    def worker(q):
+        fi = (s - 1) * t
+        yield
+        last = flags.get(fi, 0) == s - 1  # peek
+        if not last:
+            yield
+            slots[s * t + q] = "ready"
+            yield
+            count = flags.get(fi, 0)
+            flags[fi] = count + 1  # ticket
+            last = count == s - 1
+        if not last:
+            return
+        yield
+        flags[fi] = 0
+        held = {q}
+        for other in [p for p in (q ^ 1, (q & 2) ^ 2, (q & 2) ^ 3) if p < s]:
+            yield
+            assert slots.get(s * t + other) == "ready" and other not in held
+            held.add(other)
+        stored.append((t, frozenset(held)))
+
+    return [worker(q) for q in range(s)]
+
+
+@pytest.mark.parametrize("s", [2, 3, 4])
+def test_one_flag_meetings_store_each_tile_once(s):
+    for seed in range(400):
+        rng = random.Random(seed)
+        rem = rng.randint(1, 6)
+        flags, slots, stored = {}, {}, []
+        gens = [g for t in range(rem) for g in run_tile_one_flag(s, t, flags, slots, stored)]
+        alive = list(range(len(gens)))
+        while alive:
+            i = rng.choice(alive)
+            try:
+                next(gens[i])
+            except StopIteration:
+                alive.remove(i)
+        assert sorted(t for t, _ in stored) == list(range(rem))
+        assert all(held == frozenset(range(s)) for _, held in stored)
+        assert all(0 <= k < s * rem for k in slots)
+        assert all(0 <= k < (s - 1) * rem for k in flags)
+        assert all(v == 0 for v in flags.values())
